@@ -208,6 +208,7 @@ struct gsw_graph {
   gsw::ms_counters_t *ms_cnt = nullptr;
   gsw::ms_counters_t *ms_hcnt = nullptr;
   int32_t *ms_src = nullptr;
+  gsw::ms_wide_t ms_out, ms_in;  // wide rows of the out- and in-CSR
   // multi-root BFS state: roots on the device, the device level counter and
   // the captured level loop (instantiated once per launch shape)
   int32_t *d_roots = nullptr;
@@ -298,6 +299,12 @@ struct gsw_graph {
     if (ms_cnt) hipFree(ms_cnt);
     if (ms_hcnt) hipHostFree(ms_hcnt);
     if (ms_src) hipFree(ms_src);
+    for (gsw::ms_wide_t *w : {&ms_out, &ms_in}) {
+      if (w->v) hipFree(w->v);
+      if (w->ent) hipFree(w->ent);
+      if (w->acc) hipFree(w->acc);
+      if (w->cnt) hipFree(w->cnt);
+    }
   }
 };
 
@@ -2119,8 +2126,24 @@ gsw_status gsw_gc(gsw_graph *G, const gsw_run_opts *opts, int32_t *colors_out,
   });
 }
 
-// ---- selector trees ----------------------------------------------------------
 // ---- 64-source bitmask BFS ------------------------------------------------
+// The wide rows of one CSR (kernels/msbfs.h), listed once per graph.
+static void ms_wide_build(gsw_graph *G, const int64_t *rows, gsw::ms_wide_t &w) {
+  using namespace gsw;
+  if (w.cnt) return;
+  const int64_t n = G->hg.n, m = G->hg.m;
+  w.cap_v = ms_wide_cap_v(n, m);
+  w.cap_e = ms_wide_cap_e(n, m);
+  if (!w.v) H_ERR(hipMalloc((void **)&w.v, sizeof(int32_t) * w.cap_v));
+  if (!w.ent) H_ERR(hipMalloc((void **)&w.ent, sizeof(int2) * w.cap_e));
+  if (!w.acc) H_ERR(hipMalloc((void **)&w.acc, sizeof(unsigned long long) * w.cap_v));
+  H_ERR(hipMalloc((void **)&w.cnt, sizeof(unsigned long long) * 2));
+  fill_async<unsigned long long>(w.cnt, 0ull, 2);
+  hipLaunchKernelGGL(k_msbfs_wide, dim3(grid_for((n + 63) / 64 * 64)), dim3(BLOCK), 0,
+                     stream(), rows, n, w);
+  H_ERR(hipGetLastError());
+}
+
 gsw_status gsw_msbfs64(gsw_graph *G, const int32_t *sources, int32_t nsrc,
                        const gsw_run_opts *opts, uint64_t *mask_out,
                        uint64_t *level_sums_out, gsw_run_stats *stats) {
@@ -2136,9 +2159,17 @@ gsw_status gsw_msbfs64(gsw_graph *G, const int32_t *sources, int32_t nsrc,
     if (!G->ms_buf) {
       H_ERR(hipMalloc((void **)&G->ms_buf, sizeof(uint64_t) * 3 * (n + 1)));
       H_ERR(hipMalloc((void **)&G->ms_cnt, sizeof(ms_counters_t) * MS_SLOTS));
-      H_ERR(hipHostMalloc((void **)&G->ms_hcnt, sizeof(ms_counters_t) * MS_SLOTS));
+      H_ERR(hipHostMalloc((void **)&G->ms_hcnt, sizeof(ms_counters_t)));
       H_ERR(hipMalloc((void **)&G->ms_src, sizeof(int32_t) * 64));
     }
+    // (the degree statistics cover the out-degrees only)
+    const bool wide = G->hg.directed || G->attr.max_deg > MS_WIDE;
+    if (wide) {
+      ms_wide_build(G, G->dg.dg_row_ptr, G->ms_out);
+      if (G->hg.directed) ms_wide_build(G, G->dg.dgr_row_ptr, G->ms_in);
+    }
+    const ms_wide_t &wout = G->ms_out;
+    const ms_wide_t &win = G->hg.directed ? G->ms_in : G->ms_out;
     uint64_t *visit = G->ms_buf, *front = G->ms_buf + (n + 1),
              *next = G->ms_buf + 2 * (n + 1);
     const uint64_t all = (nsrc == 64) ? ~0ull : ((1ull << nsrc) - 1);
@@ -2150,6 +2181,8 @@ gsw_status gsw_msbfs64(gsw_graph *G, const int32_t *sources, int32_t nsrc,
                          hipMemcpyHostToDevice, st));
     H_ERR(hipEventRecord(G->ev0, st));
     fill_async<uint64_t>(visit, 0, 2 * (n + 1));  // visit and front
+    fill_async<unsigned long long>((unsigned long long *)G->ms_cnt, 0ull,
+                                   sizeof(ms_counters_t) / 8 * MS_SLOTS);
     hipLaunchKernelGGL(k_msbfs_seed, dim3(1), dim3(64), 0, st, visit, front,
                        (const int32_t *)G->ms_src, nsrc);
     double front_deg = 0;
@@ -2170,15 +2203,18 @@ gsw_status gsw_msbfs64(gsw_graph *G, const int32_t *sources, int32_t nsrc,
       // frontier's edges exceed 1/32 of the graph
       const bool pull = o.force.has_direction ? (o.force.d == Pull)
                                               : front_deg > (double)m / 32.0;
-      fill_async<unsigned long long>((unsigned long long *)G->ms_cnt, 0ull,
-                                     sizeof(ms_counters_t) / 8 * MS_SLOTS);
       if (pull) {
         // bottom-up over the in-edges (the reverse CSR; the same arrays
         // for an undirected graph)
+        if (wide)
+          hipLaunchKernelGGL(k_msbfs_pull_wide, dim3(grid_for(win.cap_e * WAVE)),
+                             dim3(BLOCK), 0, st, (const int64_t *)G->dg.dgr_row_ptr,
+                             (const int32_t *)G->dg.dgr_adj_list, all,
+                             (const uint64_t *)visit, (const uint64_t *)front, win);
         hipLaunchKernelGGL(k_msbfs_pull, dim3(grid), dim3(BLOCK), 0, st,
                            (const int64_t *)G->dg.dgr_row_ptr,
                            (const int32_t *)G->dg.dgr_adj_list, rows, n, all,
-                           visit, (const uint64_t *)front, next, G->ms_cnt);
+                           visit, (const uint64_t *)front, next, G->ms_cnt, wide, win);
       } else if (level == 1) {
         // the sources' edges spread over the grid (they are often hubs)
         fill_async<uint64_t>(next, 0, n + 1);
@@ -2191,21 +2227,15 @@ gsw_status gsw_msbfs64(gsw_graph *G, const int32_t *sources, int32_t nsrc,
         fill_async<uint64_t>(next, 0, n + 1);
         hipLaunchKernelGGL(k_msbfs_push, dim3(grid), dim3(BLOCK), 0, st, rows,
                            cols, n, (const uint64_t *)visit,
-                           (const uint64_t *)front, next);
+                           (const uint64_t *)front, next, wide, wout);
         hipLaunchKernelGGL(k_msbfs_sweep, dim3(grid), dim3(BLOCK), 0, st, rows,
                            n, visit, next, G->ms_cnt);
       }
+      hipLaunchKernelGGL(k_msbfs_finish, dim3(1), dim3(BLOCK), 0, st, G->ms_cnt,
+                         (unsigned long long *)G->ms_hcnt);
       H_ERR(hipGetLastError());
-      H_ERR(hipMemcpyAsync(G->ms_hcnt, G->ms_cnt, sizeof(ms_counters_t) * MS_SLOTS,
-                           hipMemcpyDeviceToHost, st));
       sync();
-      ms_counters_t tot{};
-      for (int k = 0; k < MS_SLOTS; ++k) {  // sum the partial slots
-        const ms_counters_t &p = G->ms_hcnt[k];
-        tot.newly += p.newly;
-        tot.newly_deg += p.newly_deg;
-        for (int s = 0; s < 64; ++s) tot.per_src[s] += p.per_src[s];
-      }
+      const ms_counters_t &tot = *G->ms_hcnt;
       gsw_level_record rec{};
       rec.level = level;
       rec.dir = pull ? 1 : 0;

@@ -95,3 +95,50 @@ def test_msbfs_directed(gsw, orc, direction):
         rev[orc.bfs(rrp, rcol, int(r)) >= 0] |= np.uint64(1) << np.uint64(s)
     assert not np.array_equal(rev, em)
     g.close()
+
+
+@pytest.mark.parametrize("direction", [None, "Push-x-x-x", "Pull-x-x-x"])
+@pytest.mark.parametrize("directed", [False, True])
+def test_msbfs_wide_rows(gsw, orc, direction, directed):
+    """Rows at the edges of the wide-row chunks (64, 65, 1024, 1025 and 3000
+    edges), reached at every level of a path that strings their hubs
+    together."""
+    degs = [64, 65, 1024, 1025, 3000, 63, 130]
+    src, dst, nxt = [], [], len(degs)
+    for h, d in enumerate(degs):
+        inner = d - (1 if h in (0, len(degs) - 1) else 2)  # path edges count too
+        leaves = np.arange(nxt, nxt + inner)
+        src += [h] * inner
+        dst += list(leaves)
+        nxt += inner
+        if h + 1 < len(degs):
+            src.append(h)
+            dst.append(h + 1)
+    if directed:  # leaves point at the next hub: wide in-rows as well
+        s, d = np.array(src), np.array(dst)
+        leaf = d >= len(degs)
+        src = np.concatenate([s, d[leaf]])
+        dst = np.concatenate([d, (s[leaf] + 1) % len(degs)])
+    h = gsw.from_edges(nxt, src, dst, directed=directed)
+    g = gsw.Graph(h)
+    rng = np.random.default_rng(3)
+    roots = np.concatenate([[0, 6], rng.integers(0, nxt, 62)]).astype(np.int32)
+    for _ in range(2):  # the wide rows' masks are clean again after a run
+        masks, sums = g.msbfs64(roots, configs=direction)
+        em, es = oracle_masks_and_sums(orc, h, roots)
+        assert np.array_equal(masks, em)
+        assert np.array_equal(sums, es)
+    g.close()
+
+
+def test_msbfs_more_words_than_wavefronts(gsw, orc):
+    """More 64-vertex words than resident wavefronts, so wavefronts reach the
+    wide rows while others still walk narrow ones."""
+    h = gsw.rmat(20, 4, seed=9)
+    g = gsw.Graph(h)
+    src = np.random.default_rng(4).integers(0, h.n, 64).astype(np.int32)
+    masks, sums = g.msbfs64(src, configs="Pull-x-x-x")
+    em, es = oracle_masks_and_sums(orc, h, src)
+    assert np.array_equal(masks, em)
+    assert np.array_equal(sums, es)
+    g.close()
