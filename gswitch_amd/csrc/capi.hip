@@ -217,11 +217,11 @@ struct gsw_graph {
   hipGraph_t cap_graph = nullptr;
   hipGraphExec_t cap_exec = nullptr;
   int cap_key[5] = {-1, -1, -1, -1, -1};
-  // sampled-hooking CC: labels (parent pointers), the vertex sample for the
-  // skipped component, batch instance offsets and the captured kernel
+  // sampled-hooking CC: labels (parent pointers), the root of the skipped
+  // component, batch instance offsets and the captured kernel
   // sequence of the batched form (instantiated per instance count)
   int32_t *cc_lab = nullptr;
-  int32_t *cc_ids = nullptr;   // sampled vertex ids [CC_SAMPLE] + chosen root
+  int32_t *cc_skip = nullptr;  // the chosen root
   int64_t *inst_off = nullptr;
   int64_t inst_cap = 0;
   hipGraph_t cc_graph = nullptr;
@@ -274,7 +274,7 @@ struct gsw_graph {
     if (do_hist) hipFree(do_hist);
     if (do_hctrl) hipHostFree(do_hctrl);
     if (cc_lab) hipFree(cc_lab);
-    if (cc_ids) hipFree(cc_ids);
+    if (cc_skip) hipFree(cc_skip);
     if (inst_off) hipFree(inst_off);
     if (d_roots) hipFree(d_roots);
     if (d_level) hipFree(d_level);
@@ -1020,25 +1020,26 @@ constexpr int CC_SAMPLE = 1024;
 void cc_buffers(gsw_graph *G) {
   if (G->cc_lab) return;
   H_ERR(hipMalloc((void **)&G->cc_lab, sizeof(int32_t) * (G->hg.n + 1)));
-  H_ERR(hipMalloc((void **)&G->cc_ids, sizeof(int32_t) * (CC_SAMPLE + 64)));
+  H_ERR(hipMalloc((void **)&G->cc_skip, sizeof(int32_t)));
 }
 
-// init, two sampling rounds, compress (phases 1-2) into lab[n]
-void cc_sample_phase(const gsw_graph *G, int32_t *lab, hipStream_t st) {
+// start, one sampling round, a compress after each (phases 1-2) into lab[n];
+// with `skip_lv`, only the vertices whose skip_lv entry is negative sample
+void cc_sample_phase(const gsw_graph *G, int32_t *lab, const int32_t *skip_lv,
+                     hipStream_t st) {
   using namespace gsw;
   const int64_t n = G->hg.n;
   const int grid = grid_for(n);
-  hipLaunchKernelGGL(k_cc_init, dim3(grid), dim3(BLOCK), 0, st, lab, n);
-  // a compress after each round: sampled links on a grid build chains
-  // thousands long, which the second round's links would walk (4096-square
-  // grid: 107 ms with one compress at the end, 3.3 ms with two)
-  for (int r = 0; r < 2; ++r) {
-    hipLaunchKernelGGL(k_cc_sample, dim3(grid), dim3(BLOCK), 0, st,
-                       (const int64_t *)G->dg.dg_row_ptr,
-                       (const int32_t *)G->dg.dg_adj_list, n, r, lab,
-                       (const int *)nullptr);
-    hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(BLOCK), 0, st, lab, n);
-  }
+  if (!skip_lv)
+    hipLaunchKernelGGL(k_cc_start, dim3(grid), dim3(BLOCK), 0, st,
+                       (const int32_t *)G->dg.dgr_first, lab, n);
+  // (compressed before the next links: chains on a grid are as long as its
+  // sides, and every link would walk them)
+  hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(BLOCK), 0, st, lab, n);
+  hipLaunchKernelGGL(k_cc_sample, dim3(grid), dim3(BLOCK), 0, st,
+                     (const int64_t *)G->dg.dg_row_ptr,
+                     (const int32_t *)G->dg.dg_adj_list, n, lab, (const int *)skip_lv);
+  hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(BLOCK), 0, st, lab, n);
   H_ERR(hipGetLastError());
 }
 
@@ -1050,7 +1051,7 @@ void cc_finish_phase(const gsw_graph *G, int32_t *lab, int skip_root,
   const int64_t n = G->hg.n;
   hipLaunchKernelGGL(k_cc_rest, dim3(grid_for((n + 63) / 64 * 64)), dim3(BLOCK), 0,
                      st, (const int64_t *)G->dg.dg_row_ptr,
-                     (const int32_t *)G->dg.dg_adj_list, n, 2, skip_root, skip_dev,
+                     (const int32_t *)G->dg.dg_adj_list, n, skip_root, skip_dev,
                      off, count, lab, 0);
   hipLaunchKernelGGL(k_cc_compress, dim3(grid_for(n)), dim3(BLOCK), 0, st, lab, n);
   H_ERR(hipGetLastError());
@@ -1058,30 +1059,27 @@ void cc_finish_phase(const gsw_graph *G, int32_t *lab, int skip_root,
 
 // CC of one graph into lab[n]: the skipped component is the most frequent
 // root among `samples` sampled vertices, found on the device (directed
-// graphs skip nothing: an out-edge is seen from one end only). `ids` holds
-// samples + 1 ints of scratch (the sample, then the chosen root). No host
-// read and no allocation: every launch is queued on `st`.
-void cc_sampled_launch(const gsw_graph *G, int32_t *lab, int32_t *ids, int samples,
+// graphs skip nothing: an out-edge is seen from one end only) and left in
+// *skip (device). No host read and no allocation: every launch is queued on
+// `st`.
+void cc_sampled_launch(const gsw_graph *G, int32_t *lab, int32_t *skip, int samples,
                        hipStream_t st) {
   using namespace gsw;
   if (G->hg.n == 0) return;
-  cc_sample_phase(G, lab, st);
+  cc_sample_phase(G, lab, nullptr, st);
   if (G->hg.directed) {
     cc_finish_phase(G, lab, -2, nullptr, nullptr, 1, st);
     return;
   }
-  int32_t *skip = ids + samples;
-  hipLaunchKernelGGL(k_cc_sample_ids, dim3((samples + BLOCK - 1) / BLOCK), dim3(BLOCK),
-                     0, st, ids, samples, G->hg.n);
   hipLaunchKernelGGL(k_cc_mode, dim3(1), dim3(CC_MODE_BLOCK), 0, st,
-                     (const int *)lab, (const int32_t *)ids, samples, skip);
+                     (const int *)lab, samples, G->hg.n, skip);
   H_ERR(hipGetLastError());
   cc_finish_phase(G, lab, -2, skip, nullptr, 1, st);
 }
 
 void cc_sampled_run(gsw_graph *G) {
   cc_buffers(G);
-  cc_sampled_launch(G, G->cc_lab, G->cc_ids, CC_SAMPLE, gsw::stream());
+  cc_sampled_launch(G, G->cc_lab, G->cc_skip, CC_SAMPLE, gsw::stream());
 }
 
 // Whether no edge of the graph leaves its instance (G->inst_off, count + 1
@@ -1109,8 +1107,8 @@ bool batch_disjoint(gsw_graph *G, const int64_t *offsets, int64_t count) {
 
 // Batched CC over instances no edge leaves, from the BFS levels of every
 // instance's first vertex (k_cc_seed_levels): the reached vertices are
-// labelled at once and skipped; the others are hooked (two sampled rounds,
-// then their remaining edges) and compressed.
+// labelled at once and skipped; the others are hooked (start, one sampled
+// round, then all their edges) and compressed.
 void cc_batched_from_levels(gsw_graph *G, int64_t count, const int32_t *lv) {
   using namespace gsw;
   cc_buffers(G);
@@ -1118,16 +1116,12 @@ void cc_batched_from_levels(gsw_graph *G, int64_t count, const int32_t *lv) {
   const int64_t n = G->hg.n;
   int32_t *lab = G->cc_lab;
   hipLaunchKernelGGL(k_cc_seed_levels, dim3(grid_for((n + 63) / 64 * 64)), dim3(BLOCK), 0,
-                     st, lab, (const int *)lv, (const int64_t *)G->inst_off, count, n);
-  for (int r = 0; r < 2; ++r) {
-    hipLaunchKernelGGL(k_cc_sample, dim3(grid_for(n)), dim3(BLOCK), 0, st,
-                       (const int64_t *)G->dg.dg_row_ptr,
-                       (const int32_t *)G->dg.dg_adj_list, n, r, lab, (const int *)lv);
-    hipLaunchKernelGGL(k_cc_compress, dim3(grid_for(n)), dim3(BLOCK), 0, st, lab, n);
-  }
+                     st, lab, (const int *)lv, (const int32_t *)G->dg.dgr_first,
+                     (const int64_t *)G->inst_off, count, n);
+  cc_sample_phase(G, lab, lv, st);
   hipLaunchKernelGGL(k_cc_rest, dim3(grid_for((n + 63) / 64 * 64)), dim3(BLOCK), 0, st,
                      (const int64_t *)G->dg.dg_row_ptr, (const int32_t *)G->dg.dg_adj_list,
-                     n, 2, -1, (const int *)nullptr, (const int64_t *)G->inst_off, count,
+                     n, -1, (const int *)nullptr, (const int64_t *)G->inst_off, count,
                      lab, 1);
   hipLaunchKernelGGL(k_cc_compress, dim3(grid_for(n)), dim3(BLOCK), 0, st, lab, n);
   H_ERR(hipGetLastError());
@@ -1145,7 +1139,7 @@ void cc_batched_captured(gsw_graph *G, int64_t count) {
     G->drop_cc_capture();
     H_ERR(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
     try {
-      cc_sample_phase(G, G->cc_lab, st);
+      cc_sample_phase(G, G->cc_lab, nullptr, st);
       cc_finish_phase(G, G->cc_lab, -1, nullptr, G->inst_off, count, st);
     } catch (...) {
       hipGraph_t dead = nullptr;
@@ -2822,11 +2816,11 @@ gsw_status gsw_scan_exclusive_i64(const int64_t *in, int64_t n, int64_t *out) {
 // ---- allocation-free connected components -------------------------------
 namespace {
 
-// Scratch of gsw_cc_noalloc: the sampled vertex ids, then the chosen root.
+// Scratch of gsw_cc_noalloc: the chosen root.
 // Every GPU holds its own copy for the life of the process. In host code
 // the name is only a stand-in for the symbol: kernels get the device address
 // that hipGetSymbolAddress returns for the current device.
-constexpr int NOALLOC_SCRATCH_INTS = gsw::CC_MAX_SAMPLES + 64;
+constexpr int NOALLOC_SCRATCH_INTS = 64;
 static __device__ __align__(256) int32_t scratch[NOALLOC_SCRATCH_INTS];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -2859,7 +2853,7 @@ gsw_status gsw_cc_noalloc(const gsw_graph *G, int32_t samples, int32_t *labels,
     GSW_REQUIRE(G && labels, GSW_E_INVALID, "invalid arguments");
     GSW_REQUIRE(samples >= 1 && samples <= gsw::CC_MAX_SAMPLES, GSW_E_INVALID,
                 "samples must be 1.." + std::to_string(gsw::CC_MAX_SAMPLES) +
-                    " (the size of the static scratch)");
+                    " (the size of the sample's table)");
     hipPointerAttribute_t attr;
     const hipError_t pe = hipPointerGetAttributes(&attr, labels);
     if (pe != hipSuccess) (void)hipGetLastError();  // clear the failed query

@@ -10,16 +10,16 @@
 // never waits on another lane: each failed CAS means the root it tried moved
 // to a smaller value, so the loop ends.
 //
-// Phases (a fixed sequence of launches, no host decisions in between for
-// the batched form, so it can live in a captured graph):
-//  1. p = identity;
-//  2. sampling: every vertex links its first neighbour, compress, links its
-//     second neighbour, compress;
+// Phases (a fixed sequence of launches, no host decisions in between, so it
+// can live in a captured graph):
+//  1. start: every vertex hooks under a smaller vertex it reaches over first
+//     (smallest) in-neighbours, with a plain store (k_cc_start), compress;
+//  2. sampling: every vertex links its second neighbour, compress;
 //  3. skip set S: vertices whose root is a chosen root -- the most frequent
 //     root of a vertex sample for one graph, or each instance's first vertex
 //     (its smallest id) for a disjoint batch. Vertices outside S link all
-//     their remaining edges; a vertex in S skips the edges that stay inside
-//     its instance (their other end is either in the same tree already or
+//     their edges; a vertex in S skips the edges that stay inside its
+//     instance (their other end is either in the same tree already or
 //     outside S, and then links the edge itself) and links only edges that
 //     leave its instance, so a batch whose instances share edges stays
 //     correct;
@@ -34,45 +34,102 @@ namespace gsw {
 
 constexpr int CC_WIDE = 128;  // degree above which a wavefront shares a row
 
+constexpr int CC_HALVE_AFTER = 16;  // steps of a link before it halves its path
+constexpr int CC_HOPS = 4;          // first neighbours a vertex follows at the start
+constexpr int CC_SILP = 4;          // vertices a lane samples at once
+
+// A parent pointer, possibly an old one from this XCD's L2: pointers only move
+// to smaller ancestors within a launch, so an old value is an ancestor too.
+// (Loads that are coherent over the device cost more: 2 M-vertex random graph
+// of mean degree 6, whole CC 276 against 303 us.)
 __device__ __forceinline__ int cc_get(const int *p, int64_t i) {
-  return __hip_atomic_load(p + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return __hip_atomic_load(p + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// join the trees of u and v: hook the larger root under the smaller one
-// with a CAS, walking up from the parents (two steps at a time on the
-// larger side) while neither is a root. Measured against finds that halve
-// the path as they walk (Jaiganesh and Burtscher, HPDC 2018): on a union of
-// 5000 random graphs the halving stores cost 180 ms against 74 ms for the
-// whole batched BFS + CC, and the compress after each sampling round
-// already keeps grid chains short (4096-square grid 3.3 vs 2.7 ms).
-__device__ __forceinline__ void cc_link(int u, int v, int *p) {
-  int a = cc_get(p, u), b = cc_get(p, v);
-  while (a != b) {
+// Join the trees of u and v: hook the larger root under the smaller one with
+// a CAS, walking up from the parents (two steps at a time on the larger side)
+// while neither is a root. The larger side strictly decreases: a vertex that
+// an old pointer shows as a root fails its CAS, which returns its parent.
+// A link that has walked CC_HALVE_AFTER steps halves its path as it goes on:
+// on a grid the trees of the start are strips whose links chain up over
+// thousands of strips (3000 x 2851 grid: this pass 1.9 ms without halving,
+// 0.47 ms with it), while on random graphs and R-MAT walks are short and the
+// stores of halving at once cost more than they save (the random graph above:
+// after 2 steps 1110 us, after 8 370, after 16 or never 277).
+__device__ __forceinline__ void cc_link(int a, int b, int *p) {
+  for (int step = 0; a != b; ++step) {
     const int hi = a > b ? a : b, lo = a > b ? b : a;
-    const int ph = cc_get(p, hi);
+    int ph = cc_get(p, hi);
     if (ph == lo) return;
-    if (ph == hi && atomicCAS(p + hi, hi, lo) == hi) return;
-    a = cc_get(p, cc_get(p, hi));
+    if (ph == hi) {
+      ph = atomicCAS(p + hi, hi, lo);
+      if (ph == hi) return;
+    }
+    a = cc_get(p, ph);
+    if (step >= CC_HALVE_AFTER)
+      __hip_atomic_store(p + hi, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     b = cc_get(p, lo);
   }
 }
 
-__global__ void __launch_bounds__(BLOCK) k_cc_init(int *p, int64_t n) {
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-       v += (int64_t)gridDim.x * blockDim.x)
-    p[v] = (int)v;
+// Where v hooks at the start: the smallest vertex within CC_HOPS steps over
+// first (smallest) in-neighbours, each smaller than the one before.
+__device__ __forceinline__ int cc_start_of(int v, const int32_t *__restrict__ first) {
+  int x = v;
+  for (int h = 0; h < CC_HOPS; ++h) {
+    const int y = first[x];
+    if (y < 0 || y >= x) break;
+    x = y;
+  }
+  return x;
 }
 
-// link every vertex with its r-th neighbour (with `skip_lv`, only the
+// p[v] <- a smaller vertex of v's component, or v. Plain stores: no two lanes
+// write one entry, and entries are only read by later launches. (Against an
+// identity fill and a CAS link of every first neighbour, and with k_cc_mode
+// below: CC of R-MAT 21 on the device 180 -> 73 us. Following up to 8 or 32 neighbours only shortens
+// chains that the compress shortens faster.)
+__global__ void __launch_bounds__(BLOCK)
+    k_cc_start(const int32_t *__restrict__ first, int *__restrict__ p, int64_t n) {
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
+       v += (int64_t)gridDim.x * blockDim.x)
+    p[v] = cc_start_of((int)v, first);
+}
+
+// link every vertex with its second neighbour (with `skip_lv`, only the
 // vertices whose skip_lv entry is negative)
 __global__ void __launch_bounds__(BLOCK)
     k_cc_sample(const int64_t *__restrict__ rows, const int32_t *__restrict__ cols,
-                int64_t n, int r, int *p, const int *__restrict__ skip_lv) {
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-       v += (int64_t)gridDim.x * blockDim.x) {
-    if (skip_lv && skip_lv[v] >= 0) continue;
-    const int64_t s = rows[v];
-    if (rows[v + 1] - s > r) cc_link((int)v, cols[s + r], p);
+                int64_t n, int *p, const int *__restrict__ skip_lv) {
+  const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t v0 = tid; v0 < n; v0 += stride * CC_SILP) {
+    // the vertices' loads together, then their links one after another
+    // (2 M-vertex random graph, R-MAT 21 of edge factor 4 with shuffled ids:
+    // whole CC 277 -> 257 and 223 -> 180 us against one vertex at a time)
+    int a[CC_SILP], b[CC_SILP];
+    int64_t s[CC_SILP];
+#pragma unroll
+    for (int k = 0; k < CC_SILP; ++k) {
+      const int64_t v = v0 + k * stride;
+      s[k] = -1;
+      if (v < n && !(skip_lv && skip_lv[v] >= 0)) {
+        const int64_t r = rows[v];
+        if (rows[v + 1] - r > 1) s[k] = r + 1;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < CC_SILP; ++k) a[k] = s[k] >= 0 ? cols[s[k]] : 0;
+#pragma unroll
+    for (int k = 0; k < CC_SILP; ++k) {
+      b[k] = 0;
+      if (s[k] >= 0) {
+        a[k] = cc_get(p, a[k]);
+        b[k] = cc_get(p, v0 + k * stride);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < CC_SILP; ++k) cc_link(a[k], b[k], p);
   }
 }
 
@@ -80,8 +137,8 @@ __global__ void __launch_bounds__(BLOCK)
 // stay put). Every vertex moves its own pointer to its grandparent until
 // the parent is a root; the pointers it reads are being shortened by their
 // own vertices at the same time, so a chain of length d collapses in about
-// log d steps per vertex instead of each vertex walking it alone (sampled
-// links on a grid make chains of thousands).
+// log d steps per vertex instead of each vertex walking it alone. Random
+// loads beyond the L2 bound it (several vertices per lane at once: no faster).
 __global__ void __launch_bounds__(BLOCK) k_cc_compress(int *p, int64_t n) {
   for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
        v += (int64_t)gridDim.x * blockDim.x) {
@@ -96,12 +153,13 @@ __global__ void __launch_bounds__(BLOCK) k_cc_compress(int *p, int64_t n) {
 }
 
 // ---- choosing the skipped component on the device ------------------------
-// A fixed sample of vertex ids (SplitMix64 output mix over key + (i+1)*phi,
-// scaled to [0, n) by a multiply-high: the host generators' counter RNG),
-// then the most frequent root among the sampled vertices. No host read, so
-// the whole CC is one asynchronous launch sequence.
+// The most frequent root among a fixed sample of vertices (ids from a
+// SplitMix64 output mix over key + (i+1)*phi, scaled to [0, n) by a
+// multiply-high: the host generators' counter RNG). No host read, so the
+// whole CC is one asynchronous launch sequence.
 constexpr int CC_MAX_SAMPLES = 4096;
 constexpr int CC_MODE_BLOCK = 1024;
+constexpr int CC_MODE_SLOTS = 6144;  // open addressing, at most 2/3 full
 constexpr uint64_t CC_SAMPLE_KEY = 0xCC5A3D1Eull;
 
 __device__ __forceinline__ uint64_t cc_mix64(uint64_t z) {
@@ -110,49 +168,58 @@ __device__ __forceinline__ uint64_t cc_mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-__global__ void __launch_bounds__(BLOCK)
-    k_cc_sample_ids(int32_t *ids, int k, int64_t n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= k) return;
-  const uint64_t key = cc_mix64(cc_mix64(CC_SAMPLE_KEY));
-  const uint64_t r = cc_mix64(key + (uint64_t)(i + 1) * 0x9E3779B97F4A7C15ull);
-  ids[i] = (int32_t)__umul64hi(r, (uint64_t)n);
-}
-
-// *skip <- the most frequent value of p[ids[0..k)] (ties: the smallest).
-// One workgroup of CC_MODE_BLOCK threads, 1 <= k <= CC_MAX_SAMPLES: bitonic
-// sort in LDS, then each run start measures its run and a 64-bit max of
-// (run length, INT_MAX - value) picks the winner.
+// *skip <- the most frequent root of the k sampled vertices (ties: the
+// smallest). One workgroup, 1 <= k <= CC_MAX_SAMPLES: the roots are counted in
+// an LDS hash table, equal roots of a wavefront by one atomic (most samples
+// hit the large component), then a 64-bit max of (count, INT_MAX - root) over
+// the table picks the winner. (Latency of one workgroup bounds it; a bitonic
+// sort of the samples and serial run counts took 61-88 us for 1024 samples.)
 __global__ void __launch_bounds__(CC_MODE_BLOCK)
-    k_cc_mode(const int *p, const int32_t *ids, int k, int *skip) {
-  __shared__ int s[CC_MAX_SAMPLES];
+    k_cc_mode(const int *p, int k, int64_t n, int *skip) {
+  __shared__ int s_key[CC_MODE_SLOTS], s_cnt[CC_MODE_SLOTS];
   __shared__ unsigned long long best;
-  int k2 = 1;
-  while (k2 < k) k2 <<= 1;
-  for (int i = threadIdx.x; i < k2; i += blockDim.x)
-    s[i] = i < k ? cc_get(p, ids[i]) : INT_MAX;
+  for (int i = threadIdx.x; i < CC_MODE_SLOTS; i += blockDim.x) {
+    s_key[i] = -1;
+    s_cnt[i] = 0;
+  }
   if (threadIdx.x == 0) best = 0;
-  for (int size = 2; size <= k2; size <<= 1)
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      __syncthreads();
-      for (int t = threadIdx.x; t < (k2 >> 1); t += blockDim.x) {
-        const int i = 2 * t - (t & (stride - 1)), j = i + stride;
-        const int a = s[i], b = s[j];
-        if ((a > b) == ((i & size) == 0)) {
-          s[i] = b;
-          s[j] = a;
+  __syncthreads();
+  const uint64_t key = cc_mix64(cc_mix64(CC_SAMPLE_KEY));
+  for (int i0 = threadIdx.x & ~(WAVE - 1); i0 < k; i0 += blockDim.x) {
+    const int i = i0 + lane_id();
+    int x = -1;
+    if (i < k) {
+      const uint64_t r = cc_mix64(key + (uint64_t)(i + 1) * 0x9E3779B97F4A7C15ull);
+      x = cc_get(p, (int64_t)__umul64hi(r, (uint64_t)n));
+    }
+    uint64_t todo = ballot(i < k);
+    while (todo) {
+      // the first open lane counts every lane with its root
+      const int lead = __builtin_ctzll(todo);
+      const int y = readlane(x, lead);
+      const uint64_t same = ballot(x == y) & todo;
+      todo &= ~same;
+      if (lane_id() == lead) {
+        int h = (int)(((uint32_t)y * 2654435761u) % CC_MODE_SLOTS);
+        for (;;) {
+          const int old = atomicCAS(&s_key[h], -1, y);
+          if (old == -1 || old == y) break;
+          h = h + 1 == CC_MODE_SLOTS ? 0 : h + 1;
         }
+        atomicAdd(&s_cnt[h], __popcll(same));
       }
     }
-  __syncthreads();
-  for (int i = threadIdx.x; i < k; i += blockDim.x) {
-    if (i > 0 && s[i] == s[i - 1]) continue;
-    int j = i + 1;
-    while (j < k && s[j] == s[i]) ++j;
-    const unsigned long long key =
-        ((unsigned long long)(j - i) << 32) | (unsigned)(INT_MAX - s[i]);
-    atomicMax(&best, key);
   }
+  __syncthreads();
+  unsigned long long top = 0;
+  for (int i = threadIdx.x; i < CC_MODE_SLOTS; i += blockDim.x)
+    if (s_cnt[i]) {
+      const unsigned long long c =
+          ((unsigned long long)s_cnt[i] << 32) | (unsigned)(INT_MAX - s_key[i]);
+      top = c > top ? c : top;
+    }
+  top = wave_max_any(top);
+  if (lane_id() == 0 && top) atomicMax(&best, top);
   __syncthreads();
   if (threadIdx.x == 0) *skip = INT_MAX - (int)(unsigned)(best & 0xFFFFFFFFull);
 }
@@ -185,17 +252,18 @@ __device__ __forceinline__ int64_t cc_instance_wave(const int64_t *off, int64_t 
 // by k_cc_cross) and BFS levels from every instance's first vertex: the
 // vertices the BFS reached form the component of that first vertex, the
 // smallest id of the instance, so that id is their label; every other
-// vertex starts as its own root.
+// vertex starts as in k_cc_start (its in-neighbours are unreached as well).
 __global__ void __launch_bounds__(BLOCK)
-    k_cc_seed_levels(int *p, const int *__restrict__ lv, const int64_t *__restrict__ off,
-                     int64_t count, int64_t n) {
+    k_cc_seed_levels(int *p, const int *__restrict__ lv, const int32_t *__restrict__ first,
+                     const int64_t *__restrict__ off, int64_t count, int64_t n) {
   const int lane = lane_id();
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> LOG_WAVE;
   const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> LOG_WAVE;
   for (int64_t base = wave << 6; base < n; base += nwaves << 6) {
     const int64_t v = base + lane;
     if (v < n)
-      p[v] = lv[v] >= 0 ? (int)off[cc_instance_wave(off, count, base, v)] : (int)v;
+      p[v] = lv[v] >= 0 ? (int)off[cc_instance_wave(off, count, base, v)]
+                        : cc_start_of((int)v, first);
   }
 }
 
@@ -227,13 +295,14 @@ __global__ void __launch_bounds__(BLOCK)
 // skip_root == -1: S = {v : p[v] == first vertex of v's instance} with
 // `off` the count + 1 instance offsets; skip_root == -2: no skipping. A
 // non-null skip_dev replaces skip_root by *skip_dev (written by k_cc_mode).
-// Edges [from, deg) of each row are visited (the sampled ones are done).
+// (Every edge of a row: its first one is hooked only where k_cc_start found
+// its other end smaller.)
 // One wavefront per 64 vertices; rows longer than CC_WIDE are walked by
 // the whole wavefront, one at a time. `disjoint`: no edge leaves an
 // instance (skip_root == -1), so a vertex of S links nothing.
 __global__ void __launch_bounds__(BLOCK)
     k_cc_rest(const int64_t *__restrict__ rows, const int32_t *__restrict__ cols,
-              int64_t n, int from, int skip_arg, const int *skip_dev,
+              int64_t n, int skip_arg, const int *skip_dev,
               const int64_t *__restrict__ off, int64_t count, int *p,
               int disjoint) {
   const int skip_root = skip_dev ? *skip_dev : skip_arg;
@@ -245,9 +314,8 @@ __global__ void __launch_bounds__(BLOCK)
     int64_t s = 0, e = 0, lo = 0, hi = 0;
     bool in_s = false;
     if (v < n) {
-      s = rows[v] + from;
+      s = rows[v];
       e = rows[v + 1];
-      if (s > e) s = e;
       const int root = cc_get(p, v);
       if (skip_root >= 0) {
         in_s = root == skip_root;

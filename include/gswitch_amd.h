@@ -173,8 +173,8 @@ gsw_status gsw_sssp(gsw_graph *g, int32_t root, const gsw_run_opts *opts,
                     uint32_t *dist_out, gsw_run_stats *stats);
 /* Connected components, label = smallest vertex id in the component
  * (run_cc, application/cc.cu:82-108). By default: tree hooking over the CSR
- * with subgraph sampling (two sampled neighbours per vertex, then the
- * remaining edges of every vertex outside the most frequent sampled
+ * with subgraph sampling (two neighbours per vertex, then all the
+ * edges of every vertex outside the most frequent sampled
  * component). With opts->configs set: the reference's edge-centric hooking
  * (cc.cu:15-32) + pointer jumping (src/utils/intrinsics.cuh:328-362) through
  * the level loop, honouring the pinned choices. With opts->selector 1 or 2
@@ -191,11 +191,11 @@ gsw_status gsw_cc(gsw_graph *g, const gsw_run_opts *opts, int32_t *labels_out,
  * kernels and returns; it allocates nothing, reads nothing back and
  * synchronises nothing. `samples` (1..4096; gsw_cc uses 1024) vertices
  * are sampled to pick the component whose inner edges are skipped. The
- * sample and the chosen root live in one static device array per GPU
+ * chosen root lives in one static device array per GPU
  * (GSW_CC_NOALLOC_SCRATCH_BYTES, held until the process ends) that every
  * call on that GPU shares: calls that overlap on one GPU race. */
 #define GSW_CC_NOALLOC_MAX_SAMPLES 4096
-#define GSW_CC_NOALLOC_SCRATCH_BYTES (4 * (4096 + 64))
+#define GSW_CC_NOALLOC_SCRATCH_BYTES (4 * 64)
 gsw_status gsw_cc_noalloc(const gsw_graph *g, int32_t samples, int32_t *labels,
                           void *stream);
 /* PageRank, un-normalised: pr_0 = 1-d, pr_{k+1}(v) = 1-d + d*sum pr_k(u)/deg(u),

@@ -203,6 +203,38 @@ def test_cc_sampled_hooking_shapes(gsw, orc):
     g.close()
 
 
+@pytest.mark.parametrize("shape", ["path", "path_shuffled", "strips", "isolated", "halves",
+                                   "star_high"])
+def test_cc_long_chains_and_samples(gsw, orc, shape):
+    """Walks longer than a link takes before it halves its path (paths,
+    vertical strips joined by single rungs), a sample whose roots all differ,
+    two components of one size, and a star whose hub has the largest id."""
+    rng = np.random.default_rng(6)
+    if shape in ("path", "path_shuffled"):
+        n = 20000
+        ids = np.arange(n) if shape == "path" else rng.permutation(n)
+        e = np.stack([ids[:-1], ids[1:]], 1)
+    elif shape == "strips":  # columns of a 300 x 200 grid, one rung per pair
+        r, c = 300, 200
+        n = r * c
+        at = np.arange(n).reshape(r, c)
+        col = rng.integers(1, c, 150)
+        e = np.concatenate([np.stack([at[:-1].ravel(), at[1:].ravel()], 1),
+                            np.stack([at[r - 1, col - 1], at[r - 1, col]], 1)])
+    elif shape == "isolated":
+        n, e = 6000, np.array([[5, 4000], [5999, 17]])
+    elif shape == "halves":
+        n = 4096
+        e = np.stack([np.arange(n - 2), np.arange(2, n)], 1)
+    else:
+        n = 3001
+        e = np.stack([np.full(n - 1, n - 1), np.arange(n - 1)], 1)
+    h = gsw.from_edges(n, e[:, 0], e[:, 1])
+    g = gsw.Graph(h)
+    assert np.array_equal(g.cc(), orc.cc(h.row_ptr, h.col))
+    g.close()
+
+
 # ---------------------------------------------------------------- PageRank
 def max_rel(a, b):
     return float(np.max(np.abs(a.astype(np.float64) - b) / np.abs(b)))
