@@ -23,9 +23,10 @@
 // counters live in the control block, so every captured level is the same
 // pair of launches.
 //
-// Top-down: wavefronts take 64 frontier words per step; for every non-zero
-// word its vertices' edges are walked 64 at a time (degree scan across the
-// lanes, owner found in LDS). A vertex of more than `heavy_deg` out-edges
+// Top-down: the frontier words are shared out evenly over the wavefronts (64
+// at most per step); a wavefront takes its frontier vertices 64 at a time and
+// walks their edges 64 at a time, DO_TD such steps' loads together (degree
+// scan across the lanes, owner found in LDS). A vertex of more than `heavy_deg` out-edges
 // is not walked by one wavefront: every such vertex found in a level is
 // appended to a short list, and the next top-down level splits the listed
 // vertices' edges evenly over the whole grid (prefix of their degrees
@@ -33,8 +34,15 @@
 // by their own wavefront, 64 edges per step.
 // Bottom-up: one wavefront per frontier word, one lane per target; the
 // first probe is the per-vertex copy of the first in-neighbour (coalesced),
-// then the in-row until a frontier source is found (early exit). The next
-// frontier word is the wavefront's ballot (plain store, every word written).
+// then the in-row, DO_PROBES edges at a time, until a frontier source is found
+// (early exit). The next frontier word is the wavefront's ballot (plain store,
+// every word written).
+//
+// Dependent loads bound both: with 64 words per wavefront whatever their
+// number, vertices taken word by word, and one in-edge probed at a time, BFS
+// over 300 random graphs (2.5 M vertices, 38.9 M edges) spent 2.8 ms in
+// k_do_expand, now 0.56 ms; R-MAT 22 0.44, now 0.27 ms (with heavy vertices
+// from 560 edges on instead of 4096).
 //
 // The result is the BFS level array, the same whatever the directions.
 #pragma once
@@ -52,6 +60,8 @@ constexpr int DO_HIST_W = 4;     // direction, frontier, edges, vertices
 constexpr int DO_BU = 2;         // frontier words per wavefront step (bottom-up;
                                  // R-MAT 24 level 2: 1 word 178 us, 2 words 169 us,
                                  // 4 words 251 us: the arrays leave registers)
+constexpr int DO_TD = 2;         // 64-edge steps a top-down wavefront loads at once
+constexpr int DO_PROBES = 4;     // in-edges a bottom-up lane probes at once
 
 // control block (long long words)
 enum : int {
@@ -195,14 +205,16 @@ __device__ __forceinline__ uint64_t shfl_u64(uint64_t x, int src) {
 // lane sets them with one atomicOr on the visited word and one on the next
 // frontier word, instead of two atomics per edge. A lane owns its target
 // if the word's old value lacks the bit and no lower lane of the run has
-// the same target (a target listed by two frontier vertices).
+// the same target (a target listed by two frontier vertices). `seen` is the
+// target's visited word, loaded by the caller together with those of its
+// other edges (a word that has changed since costs an atomic, no more).
 __device__ __forceinline__ void do_visit_wave(const dobfs_t &d, const do_level_t &t,
-                                              bool valid, int u, long long &nf,
-                                              long long &mf) {
+                                              bool valid, int u, uint64_t seen,
+                                              long long &nf, long long &mf) {
   const int lane = lane_id();
   const int64_t w = valid ? (int64_t)(u >> 6) : -1;
   const uint64_t b = valid ? 1ull << (u & 63) : 0ull;
-  const bool cand = valid && !(d.vis[w] & b);
+  const bool cand = valid && !(seen & b);
   if (!ballot(cand)) return;
   // runs of equal words among consecutive lanes
   const long long wp = __shfl_up((long long)w, 1, 64);
@@ -231,8 +243,24 @@ __device__ __forceinline__ void do_visit_wave(const dobfs_t &d, const do_level_t
   if (cand && !(old & b) && !(below & b)) do_found(d, t, u, nf, mf);
 }
 
+// position of the r-th (from 0) set bit of x, r < popcount(x)
+__device__ __forceinline__ int select_bit(uint64_t x, int r) {
+  int pos = 0;
+#pragma unroll
+  for (int h = 32; h > 0; h >>= 1) {
+    const int c = __popcll((x >> pos) & ((1ull << h) - 1));
+    if (r >= c) {
+      r -= c;
+      pos += h;
+    }
+  }
+  return pos;
+}
+
 __global__ void __launch_bounds__(BLOCK) k_do_expand(dobfs_t d) {
   __shared__ int s_scan[BLOCK];
+  __shared__ int s_pre[BLOCK];
+  __shared__ uint64_t s_word[BLOCK];
   __shared__ int64_t s_start[BLOCK];
   __shared__ long long sh[BLOCK / WAVE];
   const long long *ctrl = d.ctrl;
@@ -271,24 +299,32 @@ __global__ void __launch_bounds__(BLOCK) k_do_expand(dobfs_t d) {
           const int v = hcur[o];
           u = d.cols[d.rows[v] + (k - d.hpre[o])];
         }
-        do_visit_wave(d, t, ok, u, nf, mf);
+        do_visit_wave(d, t, ok, u, ok ? d.vis[u >> 6] : 0ull, nf, mf);
       }
     }
-    // the other frontier vertices: 64 words per wavefront step
-    for (int64_t w0 = wave * WAVE; w0 < d.nw; w0 += nwaves * WAVE) {
+    // The other frontier vertices: every wavefront takes its share of the
+    // words (at most 64 per step), and its frontier vertices 64 at a time
+    // whatever words they lie in, so sparse words leave no lanes idle and a
+    // mid-sized frontier reaches the whole grid.
+    const int wps = (int)MAX((int64_t)1, MIN((int64_t)WAVE, (d.nw + nwaves - 1) / nwaves));
+    for (int64_t w0 = wave * wps; w0 < d.nw; w0 += nwaves * wps) {
       const int64_t wi = w0 + lane;
-      const uint64_t word = wi < d.nw ? t.Fc[wi] : 0ull;
-      uint64_t nz = ballot(word != 0ull);
-      while (nz) {
-        const int j = __builtin_ctzll(nz);
-        nz &= nz - 1;
-        const uint64_t bits = shfl_u64(word, j);
-        const int v = (int)(((w0 + j) << 6) + lane);
-        int deg = 0;
+      const uint64_t word = lane < wps && wi < d.nw ? t.Fc[wi] : 0ull;
+      int nvert;
+      const int pre = wave_exclusive_scan(__popcll(word), nvert);
+      if (nvert == 0) continue;  // uniform
+      s_pre[off + lane] = pre;
+      s_word[off + lane] = word;
+      wave_sync();
+      for (int i0 = 0; i0 < nvert; i0 += WAVE) {
+        const int i = i0 + lane;
+        int v = 0, deg = 0;
         int64_t start = 0;
         bool alone = false;
-        if ((bits >> lane) & 1ull) {
+        if (i < nvert) {
           ++nv;
+          const int o = owner_search(&s_pre[off], WAVE, i);
+          v = (int)(((w0 + o) << 6) + select_bit(s_word[off + o], i - s_pre[off + o]));
           deg = d.odeg[v];
           if (deg > d.heavy_deg) {
             alone = hovf;  // walked below by this wavefront
@@ -303,14 +339,24 @@ __global__ void __launch_bounds__(BLOCK) k_do_expand(dobfs_t d) {
         s_scan[off + lane] = ex;
         s_start[off + lane] = start;
         wave_sync();
-        for (int j0 = 0; j0 < tot; j0 += WAVE) {
-          const int k = j0 + lane;
-          int u = 0;
-          if (k < tot) {
-            const int o = owner_search(&s_scan[off], WAVE, k);
-            u = d.cols[s_start[off + o] + (k - s_scan[off + o])];
+        for (int j0 = 0; j0 < tot; j0 += WAVE * DO_TD) {
+          int u[DO_TD];
+          uint64_t seen[DO_TD];
+#pragma unroll
+          for (int k = 0; k < DO_TD; ++k) {
+            const int j = j0 + k * WAVE + lane;
+            u[k] = 0;
+            if (j < tot) {
+              const int o = owner_search(&s_scan[off], WAVE, j);
+              u[k] = d.cols[s_start[off + o] + (j - s_scan[off + o])];
+            }
           }
-          do_visit_wave(d, t, k < tot, u, nf, mf);
+#pragma unroll
+          for (int k = 0; k < DO_TD; ++k)
+            seen[k] = j0 + k * WAVE + lane < tot ? d.vis[u[k] >> 6] : 0ull;
+#pragma unroll
+          for (int k = 0; k < DO_TD; ++k)
+            do_visit_wave(d, t, j0 + k * WAVE + lane < tot, u[k], seen[k], nf, mf);
         }
         wave_sync();
         // heavy vertices of an overflowed list: one wavefront each
@@ -324,10 +370,12 @@ __global__ void __launch_bounds__(BLOCK) k_do_expand(dobfs_t d) {
             const int64_t k = k0 + lane;
             const bool ok = k < e;
             if (ok) ++ne;
-            do_visit_wave(d, t, ok, ok ? d.cols[k] : 0, nf, mf);
+            const int u = ok ? d.cols[k] : 0;
+            do_visit_wave(d, t, ok, u, ok ? d.vis[u >> 6] : 0ull, nf, mf);
           }
         }
       }
+      wave_sync();  // s_pre and s_word are refilled by the next step
     }
   } else {
     // bottom-up: DO_BU consecutive frontier words per wavefront step, their
@@ -357,13 +405,21 @@ __global__ void __launch_bounds__(BLOCK) k_do_expand(dobfs_t d) {
           found = (t.Fc[u >> 6] >> (u & 63)) & 1ull;
           if (!found && id[j] > 1) {
             const int64_t s = d.rrows[v];
-            for (int k = 1; k < id[j]; ++k) {
-              u = d.rcols[s + k];
-              ++ne;
-              if ((t.Fc[u >> 6] >> (u & 63)) & 1ull) {
-                found = true;
-                break;
-              }
+            for (int k = 1; k < id[j] && !found; k += DO_PROBES) {
+              int x[DO_PROBES];
+              uint64_t f[DO_PROBES];
+#pragma unroll
+              for (int r = 0; r < DO_PROBES; ++r)
+                x[r] = k + r < id[j] ? d.rcols[s + k + r] : -1;
+#pragma unroll
+              for (int r = 0; r < DO_PROBES; ++r)
+                f[r] = x[r] >= 0 ? t.Fc[x[r] >> 6] : 0ull;
+#pragma unroll
+              for (int r = 0; r < DO_PROBES; ++r)
+                if (!found && x[r] >= 0) {
+                  ++ne;
+                  found = (f[r] >> (x[r] & 63)) & 1ull;
+                }
             }
           }
         }

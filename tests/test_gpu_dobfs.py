@@ -177,3 +177,53 @@ def test_device_bfs_level_records(gsw, orc, rmat14, alpha):
         assert set(dirs) == {"Push"}
     if alpha == 1e9:
         assert "Pull" in dirs
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 4097, 70001])
+def test_device_bfs_dense_and_sparse_words(gsw, orc, n):
+    """Top-down frontiers that fill every word (a star's leaves) and that set
+    one bit of some words (a path through every 37th leaf's own tail)."""
+    hubs = np.arange(1, n)
+    tail = np.arange(1, n, 37)
+    src = np.concatenate([np.zeros(n - 1, int), tail])
+    dst = np.concatenate([hubs, n + np.arange(len(tail))])
+    h = gsw.from_edges(n + len(tail), src, dst)
+    g = gsw.Graph(h)
+    with env(GSW_DO_ALPHA=1e-9):
+        for root in (0, n - 1, h.n - 1):
+            ref = orc.bfs(h.row_ptr, h.col, root)
+            assert np.array_equal(g.bfs(root, capture=4), ref)
+            recs = g.records()
+            assert [r["verts"] for r in recs] == [int((ref == L).sum())
+                                                  for L in range(len(recs))]
+    g.close()
+
+
+def test_device_bfs_bottom_up_probe_remainders(gsw, orc):
+    """Bottom-up rows of 1..19 in-edges whose only frontier source comes last,
+    and rows without one."""
+    rng = np.random.default_rng(2)
+    src, dst = [], []
+    dead, targets, front, root = 20, 40, 30, 90
+    for k in range(targets):
+        t = dead + k
+        d = rng.choice(dead, k % 20, replace=False)
+        src += list(d)
+        dst += [t] * len(d)
+        if k < 30:
+            src.append(dead + targets + k % front)
+            dst.append(t)
+    src += [root] * front
+    dst += list(range(dead + targets, dead + targets + front))
+    h = gsw.from_edges(root + 1, src, dst, directed=True)
+    g = gsw.Graph(h)
+    ref = orc.bfs(h.row_ptr, h.col, root)
+    with env(GSW_DO_ALPHA=1e9, GSW_DO_BETA=1e9):
+        assert np.array_equal(g.bfs(root, capture=4), ref)
+        recs = g.records()
+    assert recs[1]["dir"] == "Pull"
+    indeg = np.bincount(dst, minlength=h.n)
+    reached2 = ref == 2
+    left = (ref == -1) & (indeg > 0)
+    assert recs[1]["edges"] == int(indeg[reached2 | left].sum())
+    g.close()
