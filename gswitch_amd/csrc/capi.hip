@@ -12,6 +12,7 @@
 #include "gswitch/kernels/cc.h"
 #include "gswitch/kernels/dobfs.h"
 #include "gswitch/kernels/msbfs.h"
+#include "gswitch/utils/copy_out.h"
 #include "host/host_graph.h"
 
 using namespace gsw_apps;
@@ -174,6 +175,7 @@ template <typename F> struct app_ctx_t {
 };
 
 struct gsw_graph {
+  gsw::out_ref_t outs;  // this handle keeps the result rings alive
   gsw_host::HostGraph hg;
   graph_attr_t attr;
   double mean_weight = 0;
@@ -1470,9 +1472,7 @@ gsw_status gsw_bfs(gsw_graph *G, int32_t root, const gsw_run_opts *opts,
     }
     const double ms = elapsed(G);
     auto &c = *G->bfs;
-    if (levels_out)
-      H_ERR(hipMemcpy(levels_out, c.f.data.dg_wa, sizeof(int32_t) * G->hg.n,
-                      hipMemcpyDeviceToHost));
+    gsw::copy_out({{levels_out, c.f.data.dg_wa, sizeof(int32_t) * G->hg.n}});
     if (stats) {
       stats->device_ms = ms;
       stats->levels = levels;
@@ -1509,9 +1509,7 @@ gsw_status gsw_bfs_multi(gsw_graph *G, const int32_t *roots, int32_t nroots,
       collect_records(G, G->bfs->en.executor, G->bfs->as);
     }
     const double ms = elapsed(G);
-    if (levels_out)
-      H_ERR(hipMemcpy(levels_out, G->bfs->f.data.dg_wa,
-                      sizeof(int32_t) * G->hg.n, hipMemcpyDeviceToHost));
+    gsw::copy_out({{levels_out, G->bfs->f.data.dg_wa, sizeof(int32_t) * G->hg.n}});
     if (stats) {
       stats->device_ms = ms;
       stats->levels = levels;
@@ -1580,12 +1578,8 @@ gsw_status gsw_batch_bfs_cc(gsw_graph *G, const int64_t *offsets, int32_t count,
     H_ERR(hipEventRecord(G->ev1, gsw::stream()));
     const double ms = elapsed(G);
     G->records.clear();
-    if (levels_out)
-      H_ERR(hipMemcpy(levels_out, G->bfs->f.data.dg_wa, sizeof(int32_t) * G->hg.n,
-                      hipMemcpyDeviceToHost));
-    if (labels_out)
-      H_ERR(hipMemcpy(labels_out, G->cc_lab, sizeof(int32_t) * G->hg.n,
-                      hipMemcpyDeviceToHost));
+    gsw::copy_out({{levels_out, G->bfs->f.data.dg_wa, sizeof(int32_t) * G->hg.n},
+                   {labels_out, G->cc_lab, sizeof(int32_t) * G->hg.n}});
     if (stats) {
       stats->device_ms = ms;
       stats->levels = levels;
@@ -1798,13 +1792,9 @@ gsw_status gsw_bc(gsw_graph *G, int32_t root, const gsw_run_opts *opts,
                          0, st, c.f.data.dg_wa, h.data.dg_wa, n, d_lvl, d_nsp,
                          d_dep);
       H_ERR(hipGetLastError());
-      if (levels_out)
-        H_ERR(hipMemcpy(levels_out, d_lvl, sizeof(int32_t) * n,
-                        hipMemcpyDeviceToHost));
-      if (nsp_out)
-        H_ERR(hipMemcpy(nsp_out, d_nsp, sizeof(double) * n, hipMemcpyDeviceToHost));
-      if (dep_out)
-        H_ERR(hipMemcpy(dep_out, d_dep, sizeof(double) * n, hipMemcpyDeviceToHost));
+      gsw::copy_out({{levels_out, d_lvl, sizeof(int32_t) * n},
+                     {nsp_out, d_nsp, sizeof(double) * n},
+                     {dep_out, d_dep, sizeof(double) * n}});
     }
     if (stats) {
       stats->device_ms = ms;
@@ -1840,9 +1830,7 @@ gsw_status gsw_sssp(gsw_graph *G, int32_t root, const gsw_run_opts *opts,
     H_ERR(hipEventRecord(G->ev1, st));
     const double ms = elapsed(G);
     collect_records(G, c.en.executor, c.as);
-    if (dist_out)
-      H_ERR(hipMemcpy(dist_out, c.f.data.dg_wa, sizeof(uint32_t) * G->hg.n,
-                      hipMemcpyDeviceToHost));
+    gsw::copy_out({{dist_out, c.f.data.dg_wa, sizeof(uint32_t) * G->hg.n}});
     if (stats) {
       stats->device_ms = ms;
       stats->levels = levels;
@@ -1875,9 +1863,7 @@ gsw_status gsw_cc(gsw_graph *G, const gsw_run_opts *opts, int32_t *labels_out,
       H_ERR(hipEventRecord(G->ev1, st));
       const double ms = elapsed(G);
       G->records.clear();
-      if (labels_out)
-        H_ERR(hipMemcpy(labels_out, G->cc_lab, sizeof(int32_t) * G->hg.n,
-                        hipMemcpyDeviceToHost));
+      gsw::copy_out({{labels_out, G->cc_lab, sizeof(int32_t) * G->hg.n}});
       if (stats) {
         stats->device_ms = ms;
         stats->levels = 1;
@@ -1931,9 +1917,7 @@ gsw_status gsw_cc(gsw_graph *G, const gsw_run_opts *opts, int32_t *labels_out,
     H_ERR(hipEventRecord(G->ev1, st));
     const double ms = elapsed(G);
     collect_records(G, c.en.executor, c.as);
-    if (labels_out)
-      H_ERR(hipMemcpy(labels_out, c.f.data.dg_wa, sizeof(int32_t) * G->hg.n,
-                      hipMemcpyDeviceToHost));
+    gsw::copy_out({{labels_out, c.f.data.dg_wa, sizeof(int32_t) * G->hg.n}});
     if (stats) {
       stats->device_ms = ms;
       stats->levels = level;
@@ -1998,9 +1982,7 @@ gsw_status gsw_pagerank(gsw_graph *G, float damping, int32_t iters, float eps,
     const double ms = elapsed(G);
     collect_records(G, c.en.executor, c.as);
     G->last_class = o.selector != 0 ? c.en.conf.mlp_applied : -1;
-    if (pr_out)
-      H_ERR(hipMemcpy(pr_out, G->d_out_f, sizeof(float) * G->hg.n,
-                      hipMemcpyDeviceToHost));
+    gsw::copy_out({{pr_out, G->d_out_f, sizeof(float) * G->hg.n}});
     if (stats) {
       stats->device_ms = ms;
       stats->levels = levels;
@@ -2061,9 +2043,7 @@ gsw_status gsw_delta_pagerank(gsw_graph *G, float damping, double eps,
     H_ERR(hipEventRecord(G->ev1, st));
     const double ms = elapsed(G);
     collect_records(G, c.en.executor, c.as);
-    if (pr_out)
-      H_ERR(hipMemcpy(pr_out, G->d_out_f, sizeof(float) * G->hg.n,
-                      hipMemcpyDeviceToHost));
+    gsw::copy_out({{pr_out, G->d_out_f, sizeof(float) * G->hg.n}});
     if (stats) {
       stats->device_ms = ms;
       stats->levels = levels;
@@ -2113,9 +2093,7 @@ gsw_status gsw_gc(gsw_graph *G, const gsw_run_opts *opts, int32_t *colors_out,
     H_ERR(hipEventRecord(G->ev1, st));
     const double ms = elapsed(G);
     collect_records(G, c.en.executor, c.as);
-    if (colors_out)
-      H_ERR(hipMemcpy(colors_out, c.f.data.dg_ra, sizeof(int32_t) * G->hg.n,
-                      hipMemcpyDeviceToHost));
+    gsw::copy_out({{colors_out, c.f.data.dg_ra, sizeof(int32_t) * G->hg.n}});
     if (stats) {
       stats->device_ms = ms;
       stats->levels = levels;
@@ -2249,9 +2227,7 @@ gsw_status gsw_msbfs64(gsw_graph *G, const int32_t *sources, int32_t nsrc,
     }
     H_ERR(hipEventRecord(G->ev1, st));
     const double ms = elapsed(G);
-    if (mask_out)
-      H_ERR(hipMemcpy(mask_out, visit, sizeof(uint64_t) * n,
-                      hipMemcpyDeviceToHost));
+    gsw::copy_out({{mask_out, visit, sizeof(uint64_t) * n}});
     if (level_sums_out)
       for (int s = 0; s < 64; ++s) level_sums_out[s] = sums[s];
     if (stats) {
