@@ -14,7 +14,7 @@ results on the device.
 GTEPS (Graph500 convention): SSSP counts sum(deg(v), v reached)/2,
 PageRank counts m_undirected per iteration; value = total / wall time.
 roofline: the expand variant with the largest total time; achieved =
-algorithmic bytes per launch / mean launch time (hipEvent per expand).
+algorithmic bytes per launch / mean launch time (device clock per expand).
 cpu_baseline: the oracle's SPFA and FP64 PageRank on one host core
 (5 of the 50 PageRank iterations timed and scaled by 10).
 

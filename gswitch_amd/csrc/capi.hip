@@ -235,7 +235,7 @@ struct gsw_graph {
   int32_t *do_heavy = nullptr;
   int64_t *do_hpre = nullptr;
   long long *do_ctrl = nullptr;
-  long long *do_hist = nullptr;
+  long long *do_hist = nullptr;   // pinned: written by the device loop
   long long *do_hctrl = nullptr;  // pinned copy of the first control words
   hipGraph_t do_graph = nullptr;
   hipGraphExec_t do_exec = nullptr;
@@ -273,7 +273,7 @@ struct gsw_graph {
     if (do_heavy) hipFree(do_heavy);
     if (do_hpre) hipFree(do_hpre);
     if (do_ctrl) hipFree(do_ctrl);
-    if (do_hist) hipFree(do_hist);
+    if (do_hist) hipHostFree(do_hist);
     if (do_hctrl) hipHostFree(do_hctrl);
     if (cc_lab) hipFree(cc_lab);
     if (cc_skip) hipFree(cc_skip);
@@ -682,20 +682,15 @@ int bfs_captured_run(gsw_graph *G, int64_t k, LB lb, int small, int large,
     std::memcpy(G->cap_key, key, sizeof(key));
   }
 
-  int32_t *h = G->h_flag;
   for (int done = 0; done < max_levels; done += per_launch) {
     H_ERR(hipGraphLaunch(G->cap_exec, st));
-    H_ERR(hipMemcpyAsync(h, as.queue.sizes, sizeof(int32_t),
-                         hipMemcpyDeviceToHost, st));
-    H_ERR(hipMemcpyAsync(h + 1, as.dg_ctrl + CTRL_OVERFLOW, sizeof(int32_t),
-                         hipMemcpyDeviceToHost, st));
-    gsw::sync();
-    GSW_REQUIRE(h[1] == 0, GSW_E_OVERFLOW, "frontier queue overflow");
-    if (h[0] == 0) break;
+    as.report(as.queue.sizes, 1, as.dg_ctrl + CTRL_OVERFLOW, 1);
+    GSW_REQUIRE(as.h_ctrl[1] == 0, GSW_E_OVERFLOW, "frontier queue overflow");
+    if (as.h_ctrl[0] == 0) break;
   }
   H_ERR(hipEventRecord(G->ev1, st));
-  H_ERR(hipMemcpy(h, G->d_level, sizeof(int32_t), hipMemcpyDeviceToHost));
-  return h[0];
+  as.report(G->d_level, 1, nullptr, 0);
+  return as.h_ctrl[0];
 }
 
 int default_capture_grid(const gsw_graph *G) {
@@ -896,8 +891,10 @@ gsw::dobfs_t do_view(gsw_graph *G) {
     H_ERR(hipMalloc((void **)&G->do_heavy, sizeof(int32_t) * 2 * DO_HCAP));
     H_ERR(hipMalloc((void **)&G->do_hpre, sizeof(int64_t) * (DO_HCAP + 1)));
     H_ERR(hipMalloc((void **)&G->do_ctrl, sizeof(long long) * DO_TOTAL));
-    H_ERR(hipMalloc((void **)&G->do_hist, sizeof(long long) * DO_HIST * DO_HIST_W));
-    H_ERR(hipHostMalloc((void **)&G->do_hctrl, sizeof(long long) * DO_CTRL_WORDS));
+    H_ERR(hipHostMalloc((void **)&G->do_hist, sizeof(long long) * DO_HIST * DO_HIST_W));
+    // the control words, then their mark
+    H_ERR(hipHostMalloc((void **)&G->do_hctrl, sizeof(long long) * (DO_CTRL_WORDS + 1)));
+    G->do_hctrl[DO_CTRL_WORDS] = 0;
   }
   dobfs_t d;
   d.n = n;
@@ -980,9 +977,13 @@ int bfs_device_run(gsw_graph *G, int32_t root, int per_launch, int grid, int max
   bool halted = false;
   for (int done = 0; done < max_levels && !halted; done += per_launch) {
     H_ERR(hipGraphLaunch(G->do_exec, st));
-    H_ERR(hipMemcpyAsync(G->do_hctrl, G->do_ctrl, sizeof(long long) * DO_CTRL_WORDS,
-                         hipMemcpyDeviceToHost, st));
-    sync();
+    const long long seq = h[DO_CTRL_WORDS] + 1;
+    hipLaunchKernelGGL(k_report<long long>, dim3(1), dim3(64), 0, st,
+                       (const long long *)G->do_ctrl, (int)DO_CTRL_WORDS,
+                       (const long long *)nullptr, 0, G->do_hctrl,
+                       G->do_hctrl + DO_CTRL_WORDS, seq);
+    H_ERR(hipGetLastError());
+    await_mark(h + DO_CTRL_WORDS, seq, st);
     halted = h[DO_HALT] != 0;
   }
   H_ERR(hipEventRecord(G->ev1, st));
@@ -993,11 +994,8 @@ int bfs_device_run(gsw_graph *G, int32_t root, int per_launch, int grid, int max
   G->records.clear();
   const int nrec = MIN(levels, DO_HIST);
   if (nrec > 0) {
-    std::vector<long long> hv((size_t)nrec * DO_HIST_W);
-    H_ERR(hipMemcpy(hv.data(), G->do_hist, sizeof(long long) * hv.size(),
-                    hipMemcpyDeviceToHost));
     for (int L = 0; L < nrec; ++L) {
-      const long long *r = &hv[(size_t)L * DO_HIST_W];
+      const long long *r = G->do_hist + (size_t)L * DO_HIST_W;
       gsw_level_record rec{};
       rec.level = L;
       rec.dir = r[0] ? 1 : 0;
@@ -2137,6 +2135,7 @@ gsw_status gsw_msbfs64(gsw_graph *G, const int32_t *sources, int32_t nsrc,
       H_ERR(hipMalloc((void **)&G->ms_buf, sizeof(uint64_t) * 3 * (n + 1)));
       H_ERR(hipMalloc((void **)&G->ms_cnt, sizeof(ms_counters_t) * MS_SLOTS));
       H_ERR(hipHostMalloc((void **)&G->ms_hcnt, sizeof(ms_counters_t)));
+      std::memset(G->ms_hcnt, 0, sizeof(ms_counters_t));
       H_ERR(hipMalloc((void **)&G->ms_src, sizeof(int32_t) * 64));
     }
     // (the degree statistics cover the out-degrees only)
@@ -2208,10 +2207,12 @@ gsw_status gsw_msbfs64(gsw_graph *G, const int32_t *sources, int32_t nsrc,
         hipLaunchKernelGGL(k_msbfs_sweep, dim3(grid), dim3(BLOCK), 0, st, rows,
                            n, visit, next, G->ms_cnt);
       }
+      unsigned long long *mark = (unsigned long long *)G->ms_hcnt + MS_MARK;
+      const unsigned long long seq = *mark + 1;
       hipLaunchKernelGGL(k_msbfs_finish, dim3(1), dim3(BLOCK), 0, st, G->ms_cnt,
-                         (unsigned long long *)G->ms_hcnt);
+                         (unsigned long long *)G->ms_hcnt, seq);
       H_ERR(hipGetLastError());
-      sync();
+      await_mark(mark, seq, st);
       const ms_counters_t &tot = *G->ms_hcnt;
       gsw_level_record rec{};
       rec.level = level;

@@ -38,62 +38,36 @@ struct level_record_t {
   long long active, inactive;
   long long edges;         // edges inspected by the expand (device counter)
   long long verts;         // frontier vertices expanded
-  float ms;                // expand time (hipEvent)
+  float ms;                // expand time (device clock, first to last workgroup)
 };
 
 struct executor_t {
   bool profile = true;
   std::vector<level_record_t> log;
-  std::vector<hipEvent_t> ev_pool;
-  std::vector<std::pair<int, int>> ev_pairs;  // per log entry
-  int ev_next = 0;
+  double clock_khz = 0;  // device wall clock
 
-  void clear_log() {
-    log.clear();
-    ev_pairs.clear();
-    ev_next = 0;
-  }
+  void clear_log() { log.clear(); }
+  void release() { clear_log(); }
 
-  void release() {
-    for (auto e : ev_pool) hipEventDestroy(e);
-    ev_pool.clear();
-    clear_log();
-  }
-
-  hipEvent_t next_event() {
-    if (ev_next == (int)ev_pool.size()) {
-      hipEvent_t e;
-      H_ERR(hipEventCreate(&e));
-      ev_pool.push_back(e);
-    }
-    return ev_pool[ev_next++];
-  }
-
-  // Resolve event timings of all logged expands (syncs the stream).
+  // Work counters and times of all logged expands (one report).
   void finalize_log(active_set_t &as) {
-    gsw::sync();
-    for (size_t i = 0; i < log.size(); ++i) {
-      if (ev_pairs[i].first < 0) continue;
-      float ms = 0;
-      H_ERR(hipEventElapsedTime(&ms, ev_pool[ev_pairs[i].first],
-                                ev_pool[ev_pairs[i].second]));
-      log[i].ms = ms;
+    if (log.empty() || !as.dg_work_base) return;
+    if (clock_khz == 0) {
+      int dev = 0, khz = 0;
+      H_ERR(hipGetDevice(&dev));
+      H_ERR(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+      GSW_REQUIRE(khz > 0, gsw::E_HIP, "device reports no wall clock rate");
+      clock_khz = khz;
     }
-    if (!log.empty() && as.dg_work_base) {
-      const int64_t rows = std::min<int64_t>((int64_t)log.size(), WORK_ROWS);
-      hipLaunchKernelGGL(k_work_fold, dim3((rows * WORK_N + 255) / 256), dim3(256),
-                         0, gsw::stream(), as.dg_work_base, rows);
-      H_ERR(hipGetLastError());
-      gsw::sync();
-      std::vector<unsigned long long> w(rows * WORK_N);
-      H_ERR(hipMemcpy(w.data(), as.dg_work_base,
-                      sizeof(unsigned long long) * w.size(),
-                      hipMemcpyDeviceToHost));
-      for (size_t i = 0; i < log.size(); ++i) {
-        const size_t r = std::min<size_t>(i, (size_t)rows - 1);
-        log[i].edges = (long long)w[r * WORK_N + WORK_EDGES];
-        log[i].verts = (long long)w[r * WORK_N + WORK_VERTS];
-      }
+    const int64_t rows = std::min<int64_t>((int64_t)log.size(), WORK_ROWS);
+    const unsigned long long *w = as.read_work(rows);
+    for (size_t i = 0; i < log.size(); ++i) {
+      const unsigned long long *r = w + std::min<size_t>(i, (size_t)rows - 1) * WORK_N;
+      log[i].edges = (long long)r[WORK_EDGES];
+      log[i].verts = (long long)r[WORK_VERTS];
+      // (an expand without a workgroup that counted has no stamps)
+      if (profile && r[WORK_END] > ~r[WORK_BEGIN])
+        log[i].ms = (float)((double)(r[WORK_END] - ~r[WORK_BEGIN]) / clock_khz);
     }
   }
 
@@ -232,24 +206,13 @@ struct executor_t {
       // in-neighbour is a hub, far more walks end there)
       conf.pull_first = conf.conf_pruning && fets.push_workload_ratio >= 0.1;
     }
-    int e0 = -1, e1 = -1;
-    if (profile) {
-      e0 = ev_next;
-      H_ERR(hipEventRecord(next_event(), gsw::stream()));
-    }
     dispatch(as, g, f, conf, stat);
-    if (profile) {
-      e1 = ev_next;
-      H_ERR(hipEventRecord(next_event(), gsw::stream()));
-    }
     log.push_back(rec);
     if (conf.verbose) {
       std::printf("level %d frontier %lld ", rec.level, rec.frontier);
       conf.show_hints(std::cout);
       std::cout << std::endl;
     }
-    ev_pairs.push_back({e0, e1});
-
     if (conf.conf_fuse_inspect && conf.conf_centric == VC) {
       // the next queue's length: grid size for the next level, convergence
       const int out_slot = (as.queue.mode == Normal) ? (as.queue.cursor ^ 1)
@@ -413,7 +376,7 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
                                  dim3(BLOCK), 0, st, body,
                                  as.bitmap.visited.dg_bits, stat.slots());
               hipLaunchKernelGGL(k_stat_finish, dim3(1), dim3(BLOCK), 0, st, d,
-                                 stat.slots(), stat.dg_runtime_info);
+                                 stat.slots(), stat.h_runtime_info, ++stat.seq);
               H_ERR(hipGetLastError());
               // the next frontier becomes `active`; the old active words
               // (vertices reached earlier) become the `visited` marks

@@ -1,8 +1,8 @@
 // inspector_t: the per-level "inspect" actor.
 // Follows inspector_t (src/abstraction/inspector.cuh:112-244): skip the pass
 // in fused mode and in the first round (features are synthesised from the
-// root), otherwise run the inspector kernel, read the six counters back
-// (one pinned copy + one stream sync) and turn them into features; declare
+// root), otherwise run the inspector kernel, wait for its six counters
+// (pinned host memory, polled) and turn them into features; declare
 // convergence when nothing is active (or, for idempotent algorithms, when
 // nothing is left inactive).
 #pragma once
@@ -113,7 +113,7 @@ struct inspector_t {
                          dim3(gsw::BLOCK), 0, gsw::stream(), as, g, f,
                          stat.slots());
       hipLaunchKernelGGL(gsw::k_stat_finish, dim3(1), dim3(gsw::BLOCK), 0,
-                         gsw::stream(), d, stat.slots(), stat.dg_runtime_info);
+                         gsw::stream(), d, stat.slots(), stat.h_runtime_info, ++stat.seq);
       H_ERR(hipGetLastError());
       stat.collect();
       if (d.w) conf.mlp_class = (int)stat.h_runtime_info[6];
@@ -142,7 +142,7 @@ struct inspector_t {
                        stat.slots());
     hipLaunchKernelGGL(gsw::k_stat_finish, dim3(1), dim3(gsw::BLOCK), 0,
                        gsw::stream(), gsw_mlp::sel_dev_t{}, stat.slots(),
-                       stat.dg_runtime_info);
+                       stat.h_runtime_info, ++stat.seq);
     H_ERR(hipGetLastError());
     stat.collect();
     set_fets(as, stat, fets, conf, (double)g.nvertexs, (double)g.nedges);

@@ -6,14 +6,15 @@
 // scanned edges) and the maxima are true maxima (the reference block-sums
 // them, inspector.cuh:101-109).
 //
-// Device layout: `dg_runtime_info[0..8)` holds the reduced counters the host
-// copies back; after it come STAT_SLOTS partial slots, one 128-byte line
-// each, that the counting passes add into (workgroup b uses slot
+// Device layout: STAT_SLOTS partial slots, one 128-byte line each, that the
+// counting passes add into (workgroup b uses slot
 // b % STAT_SLOTS). Atomics from every workgroup onto one line serialise at
 // about 12 ns each on MI355X (2048 workgroups x 6 counters = 150 us), while
 // the same atomics spread over 64 lines cost nothing measurable. The
-// one-workgroup finish kernel (k_stat_finish) sums the slots into the
-// reduced counters and clears them, so the slots are zero between passes.
+// one-workgroup finish kernel (k_stat_finish) sums the slots into
+// `h_runtime_info` (pinned host memory: six counters, the learned class and a
+// mark that the host polls for) and clears them, so the slots are zero
+// between passes.
 #pragma once
 #include "../model/class_tree.h"
 #include "../model/mlp.h"
@@ -23,9 +24,10 @@ constexpr int STAT_SLOTS = 64;   // partial-counter slots
 constexpr int STAT_STRIDE = 16;  // long longs per slot (one 128-byte line)
 
 struct stat_t {
-  enum { N = 8, SLOT_BASE = 16, TOTAL = SLOT_BASE + STAT_SLOTS * STAT_STRIDE };
-  long long *dg_runtime_info = nullptr;
+  enum { N = 8, MARK = 7, TOTAL = STAT_SLOTS * STAT_STRIDE };
+  long long *dg_slots = nullptr;
   long long *h_runtime_info = nullptr;
+  long long seq = 0;  // mark of the latest finish kernel
   int size = 6;
 
   // history (wall-clock ms per phase)
@@ -46,17 +48,18 @@ struct stat_t {
 
   void build(int _size = 6) {
     size = _size;
-    if (!dg_runtime_info) {
-      H_ERR(hipMalloc((void **)&dg_runtime_info, sizeof(long long) * TOTAL));
+    if (!dg_slots) {
+      H_ERR(hipMalloc((void **)&dg_slots, sizeof(long long) * TOTAL));
       H_ERR(hipHostMalloc((void **)&h_runtime_info, sizeof(long long) * N));
+      h_runtime_info[MARK] = 0;
+      gsw::fill_async<long long>(dg_slots, 0, TOTAL);
     }
-    for (int i = 0; i < N; ++i) h_runtime_info[i] = 0;
-    clean();
+    for (int i = 0; i < MARK; ++i) h_runtime_info[i] = 0;
   }
   void release() {
-    if (dg_runtime_info) hipFree(dg_runtime_info);
+    if (dg_slots) hipFree(dg_slots);
     if (h_runtime_info) hipHostFree(h_runtime_info);
-    dg_runtime_info = nullptr;
+    dg_slots = nullptr;
     h_runtime_info = nullptr;
   }
   // new run: history cleared, rule trees until a network is installed
@@ -70,19 +73,9 @@ struct stat_t {
     tree = nullptr;
   }
   // partial slots the counting passes add into
-  long long *slots() const { return dg_runtime_info + SLOT_BASE; }
-  // enqueue the device->host copy; the caller synchronises
-  void collect_async(int num = N) {
-    H_ERR(hipMemcpyAsync(h_runtime_info, dg_runtime_info,
-                         sizeof(long long) * num, hipMemcpyDeviceToHost,
-                         gsw::stream()));
-  }
-  void collect(int num = N) {
-    collect_async(num);
-    gsw::sync();
-  }
-  // zero the reduced counters and every slot
-  void clean() { gsw::fill_async<long long>(dg_runtime_info, 0, TOTAL); }
+  long long *slots() const { return dg_slots; }
+  // until the latest finish kernel's counters are on the host
+  void collect() { gsw::await_mark(h_runtime_info + MARK, seq, gsw::stream()); }
 
   long long active_num() const { return h_runtime_info[0]; }
   long long unactive_num() const { return h_runtime_info[1]; }

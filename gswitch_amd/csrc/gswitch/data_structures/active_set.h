@@ -75,24 +75,27 @@ __global__ void __launch_bounds__(256)
 }
 
 enum : int { CTRL_HALT = 0, CTRL_OVERFLOW = 1, CTRL_FLAG = 2, CTRL_N = 8 };
-// Per-expand work counters (edges scanned, vertices expanded): one record
-// row of WORK_N counters per expand, WORK_ROWS rows per traversal, kept as
+// Per-expand work counters (edges scanned, vertices expanded, and the device
+// clock at the expand's first and last workgroup: the begin stored inverted,
+// so that a maximum over zeroed rows gives both): one record row of WORK_N
+// counters per expand, WORK_ROWS rows per traversal, kept as
 // WORK_SLOTS partial copies laid out slot-major ([slot][row][counter]) so
 // that the slots of one row sit on different cache lines. k_work_fold sums
 // the slots into slot 0 when the records are read.
-enum : int { WORK_EDGES = 0, WORK_VERTS = 1, WORK_N = 4 };
+enum : int { WORK_EDGES = 0, WORK_VERTS = 1, WORK_BEGIN = 2, WORK_END = 3, WORK_N = 4 };
 constexpr int WORK_ROWS = 16384;  // per-expand counter rows kept per traversal
 constexpr int WORK_SLOTS = 16;
 constexpr int64_t WORK_SLOT_STRIDE = (int64_t)WORK_ROWS * WORK_N;
 constexpr int64_t WORK_TOTAL = WORK_SLOT_STRIDE * WORK_SLOTS;
 
 // A traversal's reset in one launch: zeroes the three frontier bitmaps
-// (n_bits words each), the control block, the work counters and the first
-// nq queue lengths; n_all is the largest of these counts.
+// (n_bits words each), the control block, the first n_work words of every
+// work slot and the first nq queue lengths; n_all is the largest of these
+// counts.
 __global__ void __launch_bounds__(256)
     k_reset_frontier(uint64_t *visited, uint64_t *active, uint64_t *inactive,
                      int64_t n_bits, int32_t *ctrl, unsigned long long *work,
-                     int32_t *qsizes, int64_t nq, int64_t n_all) {
+                     int64_t n_work, int32_t *qsizes, int64_t nq, int64_t n_all) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_all;
        i += (int64_t)gridDim.x * blockDim.x) {
     if (i < n_bits) {
@@ -101,7 +104,8 @@ __global__ void __launch_bounds__(256)
       inactive[i] = 0;
     }
     if (i < CTRL_N) ctrl[i] = 0;
-    if (i < WORK_TOTAL) work[i] = 0;
+    if (i < n_work)
+      for (int s = 0; s < WORK_SLOTS; ++s) work[s * WORK_SLOT_STRIDE + i] = 0;
     if (i < nq) qsizes[i] = 0;
   }
 }
@@ -122,18 +126,26 @@ __global__ void __launch_bounds__(64)
   if (s < WORK_SLOTS) row[s * WORK_SLOT_STRIDE + k] = 0;
 }
 
-// slot 0 of rows [0, nrows) := the sum over the slots; the other slots are
-// cleared, so folding again changes nothing
-__global__ void __launch_bounds__(256)
-    k_work_fold(unsigned long long *base, int64_t nrows) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nrows * WORK_N) return;
-  unsigned long long t = base[i];
-  for (int s = 1; s < WORK_SLOTS; ++s) {
-    t += base[s * WORK_SLOT_STRIDE + i];
-    base[s * WORK_SLOT_STRIDE + i] = 0;
+// The slots of rows [0, nrows) combined into `out` (pinned host memory) and
+// cleared; one workgroup, then the mark.
+__global__ void __launch_bounds__(1024)
+    k_work_fold(unsigned long long *base, int64_t nrows, unsigned long long *out,
+                unsigned long long *mark, unsigned long long seq) {
+  for (int64_t i = threadIdx.x; i < nrows * WORK_N; i += blockDim.x) {
+    const bool sum = i % WORK_N < WORK_BEGIN;
+    unsigned long long x[WORK_SLOTS], t = 0;
+#pragma unroll
+    for (int s = 0; s < WORK_SLOTS; ++s) x[s] = base[s * WORK_SLOT_STRIDE + i];
+#pragma unroll
+    for (int s = 0; s < WORK_SLOTS; ++s) {
+      t = sum ? t + x[s] : (x[s] > t ? x[s] : t);
+      base[s * WORK_SLOT_STRIDE + i] = 0;
+    }
+    out[i] = t;
   }
-  base[i] = t;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) gsw::publish(mark, seq);
 }
 
 struct active_set_t {
@@ -148,7 +160,12 @@ struct active_set_t {
   unsigned long long *dg_work = nullptr;      // counters of the current expand
   unsigned long long *dg_work_base = nullptr; // [WORK_SLOTS][WORK_ROWS][WORK_N]
   int32_t *dg_block_count = nullptr;          // sorted-filter scratch [1025]
-  int32_t *h_ctrl = nullptr;                  // pinned mirror of dg_ctrl
+  int32_t *h_ctrl = nullptr;                  // pinned: reported words, mark
+  enum { H_MARK = 16, H_WORDS = 32 };
+  int32_t h_seq = 0;                          // mark of the last report
+  int work_rows = 0;                          // rows written since their last clear
+  unsigned long long *h_work = nullptr;       // pinned: folded rows, then a mark
+  int64_t h_work_rows = 0;
   // host-side counts of the current frontier (from the inspector's
   // counters, or the root): the filter sizes its output queue with them
   // without a device round trip
@@ -162,7 +179,9 @@ struct active_set_t {
     H_ERR(hipMalloc((void **)&dg_ctrl, sizeof(int32_t) * CTRL_N));
     H_ERR(hipMalloc((void **)&dg_work_base, sizeof(unsigned long long) * WORK_TOTAL));
     dg_work = dg_work_base;
-    H_ERR(hipHostMalloc((void **)&h_ctrl, sizeof(int32_t) * CTRL_N));
+    work_rows = WORK_ROWS;
+    H_ERR(hipHostMalloc((void **)&h_ctrl, sizeof(int32_t) * H_WORDS));
+    h_ctrl[H_MARK] = 0;
     bytes += queue.build(n, qmode, dg_ctrl + CTRL_OVERFLOW);
     bytes += bitmap.build(n);
     reset();
@@ -178,6 +197,9 @@ struct active_set_t {
     hipFree(dg_work_base);
     if (dg_block_count) hipFree(dg_block_count);
     hipHostFree(h_ctrl);
+    if (h_work) hipHostFree(h_work);
+    h_work = nullptr;
+    h_work_rows = 0;
     dg_ctrl = nullptr;
     dg_work = dg_work_base = nullptr;
     dg_block_count = nullptr;
@@ -204,11 +226,14 @@ struct active_set_t {
     const int64_t nb = bitmap.visited.n_words + 1;
     GSW_REQUIRE(bitmap.active.n_words + 1 == nb && bitmap.inactive.n_words + 1 == nb,
                 gsw::E_INTERNAL_CHECK, "frontier bitmaps of different sizes");
-    const int64_t n_all = std::max(std::max(nb, nq), std::max((int64_t)CTRL_N, WORK_TOTAL));
+    // (a captured loop counts into row 0 without selecting it)
+    const int64_t n_work = (int64_t)std::max(work_rows, 1) * WORK_N;
+    work_rows = 0;
+    const int64_t n_all = std::max(std::max(nb, nq), std::max((int64_t)CTRL_N, n_work));
     hipLaunchKernelGGL(k_reset_frontier, dim3(gsw::grid_for(n_all, 256)), dim3(256),
                        0, gsw::stream(), bitmap.visited.dg_bits,
                        bitmap.active.dg_bits, bitmap.inactive.dg_bits, nb, dg_ctrl,
-                       dg_work_base, queue.sizes, nq, n_all);
+                       dg_work_base, n_work, queue.sizes, nq, n_all);
     H_ERR(hipGetLastError());
     dg_work = dg_work_base;
     converged = false;
@@ -265,26 +290,53 @@ struct active_set_t {
   }
   int64_t get_size_host_cached() const { return size_cached; }
 
+  // Words of device memory to h_ctrl[0..), one launch and a polled mark.
+  void report(const int32_t *a, int na, const int32_t *b, int nb) {
+    hipStream_t st = gsw::stream();
+    if (++h_seq == 0) h_seq = 1;
+    hipLaunchKernelGGL(gsw::k_report<int32_t>, dim3(1), dim3(64), 0, st, a, na, b, nb,
+                       h_ctrl, h_ctrl + H_MARK, h_seq);
+    H_ERR(hipGetLastError());
+    gsw::await_mark(h_ctrl + H_MARK, h_seq, st);
+  }
+
   // Read the device queue length of `slot` together with the control block
-  // (one stream sync); raises on a queue overflow.
+  // (one report); raises on a queue overflow.
   int read_qsize_device(int slot) {
-    int32_t *h = h_ctrl;
-    H_ERR(hipMemcpyAsync(h, dg_ctrl, sizeof(int32_t) * CTRL_FLAG,
-                         hipMemcpyDeviceToHost, gsw::stream()));
-    H_ERR(hipMemcpyAsync(h + CTRL_FLAG, queue.sizes + slot, sizeof(int32_t),
-                         hipMemcpyDeviceToHost, gsw::stream()));
-    gsw::sync();
-    queue.host_sizes[slot] = h[CTRL_FLAG];
-    GSW_REQUIRE(h[CTRL_OVERFLOW] == 0, gsw::E_OVERFLOW, "frontier queue overflow");
-    return h[CTRL_FLAG];
+    report(dg_ctrl, CTRL_FLAG, queue.sizes + slot, 1);
+    queue.host_sizes[slot] = h_ctrl[CTRL_FLAG];
+    GSW_REQUIRE(h_ctrl[CTRL_OVERFLOW] == 0, gsw::E_OVERFLOW, "frontier queue overflow");
+    return h_ctrl[CTRL_FLAG];
   }
 
   void check_overflow() {
-    H_ERR(hipMemcpyAsync(h_ctrl, dg_ctrl, sizeof(int32_t) * CTRL_FLAG,
-                         hipMemcpyDeviceToHost, gsw::stream()));
-    gsw::sync();
+    report(dg_ctrl, CTRL_FLAG, nullptr, 0);
     GSW_REQUIRE(h_ctrl[CTRL_OVERFLOW] == 0, gsw::E_OVERFLOW,
                 "frontier queue overflow");
+  }
+
+  // The work counters of the first `rows` record rows, folded (pinned host
+  // memory, rows * WORK_N words; valid until the next call).
+  const unsigned long long *read_work(int64_t rows) {
+    if (rows > h_work_rows) {
+      if (h_work) H_ERR(hipHostFree(h_work));
+      h_work = nullptr;
+      h_work_rows = 0;
+      int64_t cap = 64;
+      while (cap < rows) cap *= 2;
+      H_ERR(hipHostMalloc((void **)&h_work, sizeof(unsigned long long) * (cap * WORK_N + 8)));
+      h_work[cap * WORK_N] = 0;
+      h_work_rows = cap;
+    }
+    hipStream_t st = gsw::stream();
+    unsigned long long *mark = h_work + h_work_rows * WORK_N;
+    const unsigned long long seq = *mark + 1;
+    hipLaunchKernelGGL(k_work_fold, dim3(1), dim3(1024), 0, st, dg_work_base, rows, h_work,
+                       mark, seq);
+    H_ERR(hipGetLastError());
+    gsw::await_mark(mark, seq, st);
+    if (rows >= work_rows) work_rows = 0;
+    return h_work;
   }
   // overflow state as of the last read_qsize_device (no extra sync)
   void check_overflow_cached() const {
@@ -301,7 +353,9 @@ struct active_set_t {
   }
 
   void select_work_row(int i) {
-    dg_work = dg_work_base + (int64_t)(i < WORK_ROWS ? i : WORK_ROWS - 1) * WORK_N;
+    const int row = i < WORK_ROWS ? i : WORK_ROWS - 1;
+    dg_work = dg_work_base + (int64_t)row * WORK_N;
+    work_rows = std::max(work_rows, row + 1);
     // past the last row every expand reuses it: start it from zero
     if (i >= WORK_ROWS - 1) {
       hipLaunchKernelGGL(k_work_clear_row, dim3(1), dim3(64), 0, gsw::stream(),

@@ -86,9 +86,7 @@ bool active_set_t::finish(G &g, F &f, config_t &conf) {
                        dim3(gsw::BLOCK), 0, gsw::stream(), g, f,
                        dg_ctrl + CTRL_FLAG);
     H_ERR(hipGetLastError());
-    H_ERR(hipMemcpyAsync(h_ctrl + CTRL_FLAG, dg_ctrl + CTRL_FLAG,
-                         sizeof(int32_t), hipMemcpyDeviceToHost, gsw::stream()));
-    gsw::sync();
+    report(dg_ctrl, CTRL_FLAG + 1, nullptr, 0);
     if (h_ctrl[CTRL_FLAG]) {
       converged = false;
       window_moved = true;

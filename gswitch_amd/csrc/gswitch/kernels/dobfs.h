@@ -97,6 +97,7 @@ struct dobfs_t {
   int64_t *hpre = nullptr;         // [DO_HCAP + 1] degree prefix of the list
   long long *ctrl = nullptr;       // [DO_TOTAL]
   long long *hist = nullptr;       // [DO_HIST][DO_HIST_W] per-level history
+                                   // (pinned host memory)
   int heavy_deg = 4096;
   float alpha = 14.f, beta = 24.f;
 };
@@ -475,6 +476,7 @@ __global__ void __launch_bounds__(DO_DECIDE_BLOCK) k_do_decide(dobfs_t d) {
       hrow[1] = ctrl[DO_NF];
       hrow[2] = ne;
       hrow[3] = nv;
+      __threadfence_system();
     }
     if (nf == 0) {
       ctrl[DO_HALT] = 1;

@@ -91,6 +91,7 @@ template <typename G, typename F> struct pull_body {
 // ---------------------------------------------------------------- TM
 template <class B>
 __global__ void __launch_bounds__(BLOCK) k_pull_tm(B body) {
+  const unsigned long long t0 = wall_clock64();
   using WA = typename B::WA;
   const int64_t N = body.as.get_size();
   const Status want = body.conf.want();
@@ -136,7 +137,7 @@ __global__ void __launch_bounds__(BLOCK) k_pull_tm(B body) {
     ne += j - s;
     if (any) *body.f.wa_of(v) = acc;
   }
-  add_work(body.as.dg_work, ne, nv);
+  add_work(body.as.dg_work, t0, ne, nv);
 }
 
 // TM pull over a bitmap frontier with the next level's inspection folded
@@ -150,6 +151,7 @@ __global__ void __launch_bounds__(BLOCK) k_pull_tm(B body) {
 template <class B>
 __global__ void __launch_bounds__(BLOCK)
     k_pull_tm_inspect(B body, uint64_t *next_active, long long *slots) {
+  const unsigned long long t0 = wall_clock64();
   using WA = typename B::WA;
   __shared__ long long sh[BLOCK / WAVE];
   const int lane = lane_id();
@@ -231,12 +233,13 @@ __global__ void __launch_bounds__(BLOCK)
   flush_sum(pullw, sh, slot + 3);
   flush_max(maxa, sh, slot + 4);
   flush_max(maxi, sh, slot + 5);
-  add_work(body.as.dg_work, ne, nv);
+  add_work(body.as.dg_work, t0, ne, nv);
 }
 
 // ---------------------------------------------------------------- WM
 template <class B>
 __global__ void __launch_bounds__(BLOCK) k_pull_wm(B body) {
+  const unsigned long long t0 = wall_clock64();
   using WA = typename B::WA;
   __shared__ int s_v[BLOCK];
   __shared__ int s_scan[BLOCK];
@@ -308,12 +311,13 @@ __global__ void __launch_bounds__(BLOCK) k_pull_wm(B body) {
     }
     wave_sync();
   }
-  add_work(body.as.dg_work, ne, nv);
+  add_work(body.as.dg_work, t0, ne, nv);
 }
 
 // ---------------------------------------------------------------- CM
 template <class B>
 __global__ void __launch_bounds__(BLOCK) k_pull_cm(B body) {
+  const unsigned long long t0 = wall_clock64();
   using WA = typename B::WA;
   __shared__ int s_v[BLOCK];
   __shared__ int s_scan[BLOCK];
@@ -367,7 +371,7 @@ __global__ void __launch_bounds__(BLOCK) k_pull_cm(B body) {
       __syncthreads();
     }
   }
-  add_work(body.as.dg_work, ne, nv);
+  add_work(body.as.dg_work, t0, ne, nv);
 }
 
 // ---------------------------------------------------------------- STRICT
@@ -383,6 +387,7 @@ __device__ __forceinline__ void pull_strict_range(B &body, const slots_t sl,
                                                   const int32_t *tgt, int64_t N,
                                                   int64_t bi, int64_t nb,
                                                   bool allow_whole) {
+  const unsigned long long t0 = wall_clock64();
   using WA = typename B::WA;
   __shared__ int64_t s_scan[SCHUNK + 1];
   __shared__ int64_t s_start[SCHUNK + 1];
@@ -457,7 +462,7 @@ __device__ __forceinline__ void pull_strict_range(B &body, const slots_t sl,
     __syncthreads();
     k0 = nk;
   }
-  add_work(body.as.dg_work, ne, 0);
+  add_work(body.as.dg_work, t0, ne, 0);
 }
 
 // ------------------------------------------------- merge-path from-all pull
@@ -485,6 +490,7 @@ __device__ __forceinline__ void pull_mp_range(B &body, const int64_t *rows,
                                               const int32_t *tgt, int64_t N,
                                               int64_t bi, int64_t nb,
                                               bool exclusive) {
+  const unsigned long long t0 = wall_clock64();
   using WA = typename B::WA;
   __shared__ int s_row[MP_TILE + 2];  // row prefix relative to the tile start
   __shared__ WA s_msg[MP_TILE];
@@ -617,7 +623,7 @@ __device__ __forceinline__ void pull_mp_range(B &body, const int64_t *rows,
     __syncthreads();
     k0 = nk;
   }
-  add_work(body.as.dg_work, ne, 0);
+  add_work(body.as.dg_work, t0, ne, 0);
 }
 
 template <class B>
@@ -758,6 +764,7 @@ __device__ __forceinline__ unsigned long long pull_bin_chunks(
 // last blocks[2] the chunks of the longer rows
 template <class B>
 __global__ void __launch_bounds__(BLOCK) k_pull_bins(B body, twod_slice_t sl) {
+  const unsigned long long t0 = wall_clock64();
   static_assert(TWOD_BINS == 2, "two row bins and the chunks");
   int64_t b = blockIdx.x;
   unsigned long long ne = 0;
@@ -771,7 +778,7 @@ __global__ void __launch_bounds__(BLOCK) k_pull_bins(B body, twod_slice_t sl) {
     b -= sl.blocks[1];
     ne = pull_bin_chunks(body, sl, b, sl.blocks[2]);
   }
-  add_work(body.as.dg_work, ne, 0);
+  add_work(body.as.dg_work, t0, ne, 0);
 }
 
 template <class B>

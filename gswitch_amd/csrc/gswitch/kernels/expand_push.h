@@ -30,14 +30,25 @@
 
 namespace gsw {
 
-// Edge / vertex work counters of an expand: a workgroup reduction, then one
-// atomic per counter into the workgroup's slot of the current record row
-// (slot blockIdx.x % WORK_SLOTS; the slots of a row lie WORK_ROWS rows
-// apart, so each has a cache line of its own: atomics from every workgroup
-// onto one line serialise on MI355X). Every thread of the workgroup calls
-// it; a workgroup that leaves early leaves as a whole and counts nothing.
+// Edge / vertex work counters of an expand and its clock stamps: a workgroup
+// reduction, then one atomic per counter into the workgroup's slot of the
+// current record row (slot blockIdx.x % WORK_SLOTS; the slots of a row lie
+// WORK_ROWS rows apart, so each has a cache line of its own: atomics from
+// every workgroup onto one line serialise on MI355X). Every thread of the
+// workgroup calls it; a workgroup that leaves early leaves as a whole and
+// counts nothing. `t0`: the device clock when the kernel began. (Stamps
+// instead of an event before and after every expand: an event pair costs the
+// stream 7 us, a third of a small PageRank iteration.)
+__device__ __forceinline__ unsigned long long *work_slot(unsigned long long *work) {
+  return work + (int64_t)(blockIdx.x & (WORK_SLOTS - 1)) * WORK_SLOT_STRIDE;
+}
+// the begin of an expand of several launches, in its first one
+__device__ __forceinline__ void stamp_begin(unsigned long long *work) {
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    atomicMax(work + WORK_BEGIN, ~(unsigned long long)wall_clock64());
+}
 template <int NT = BLOCK>
-__device__ __forceinline__ void add_work(unsigned long long *work,
+__device__ __forceinline__ void add_work(unsigned long long *work, unsigned long long t0,
                                          unsigned long long edges,
                                          unsigned long long verts) {
   __shared__ unsigned long long sh[2][NT / WAVE];
@@ -55,10 +66,12 @@ __device__ __forceinline__ void add_work(unsigned long long *work,
       e += sh[0][i];
       v += sh[1][i];
     }
-    unsigned long long *slot =
-        work + (int64_t)(blockIdx.x & (WORK_SLOTS - 1)) * WORK_SLOT_STRIDE;
+    unsigned long long *slot = work_slot(work);
     if (e) atomicAdd(slot + WORK_EDGES, e);
     if (v) atomicAdd(slot + WORK_VERTS, v);
+    // workgroups start in order: the first one of each slot begins it
+    if (blockIdx.x < WORK_SLOTS) atomicMax(slot + WORK_BEGIN, ~t0);
+    atomicMax(slot + WORK_END, (unsigned long long)wall_clock64());
   }
 }
 
@@ -118,6 +131,7 @@ template <typename G, typename F, bool FUSED> struct push_body {
 // ---------------------------------------------------------------- TM
 template <class B>
 __global__ void __launch_bounds__(BLOCK) k_push_tm(B body) {
+  const unsigned long long t0 = wall_clock64();
   __shared__ int s_stage[B::STAGE_LDS];
   auto st = body.stage(s_stage);
   const int lane = lane_id();
@@ -149,7 +163,7 @@ __global__ void __launch_bounds__(BLOCK) k_push_tm(B body) {
     }
   }
   body.emit_flush(st, s_stage);
-  add_work(body.as.dg_work, ne, nv);
+  add_work(body.as.dg_work, t0, ne, nv);
 }
 
 // ---------------------------------------------------------------- WM
@@ -158,6 +172,7 @@ template <class B>
 // edges 64 at a time: with a small mean degree fewer items per wavefront
 // means more wavefronts in flight and fewer dependent 64-edge steps each.
 __global__ void __launch_bounds__(BLOCK) k_push_wm(B body, int vpw) {
+  const unsigned long long t0 = wall_clock64();
   __shared__ int s_stage[B::STAGE_LDS];
   auto st = body.stage(s_stage);
   __shared__ int s_v[BLOCK];
@@ -202,12 +217,13 @@ __global__ void __launch_bounds__(BLOCK) k_push_wm(B body, int vpw) {
     wave_sync();
   }
   body.emit_flush(st, s_stage);
-  add_work(body.as.dg_work, ne, nv);
+  add_work(body.as.dg_work, t0, ne, nv);
 }
 
 // ---------------------------------------------------------------- CM
 template <class B>
 __global__ void __launch_bounds__(BLOCK) k_push_cm(B body) {
+  const unsigned long long t0 = wall_clock64();
   __shared__ int s_stage[B::STAGE_LDS];
   auto st = body.stage(s_stage);
   __shared__ int s_v[BLOCK];
@@ -250,7 +266,7 @@ __global__ void __launch_bounds__(BLOCK) k_push_cm(B body) {
     __syncthreads();
   }
   body.emit_flush(st, s_stage);
-  add_work(body.as.dg_work, ne, nv);
+  add_work(body.as.dg_work, t0, ne, nv);
 }
 
 // ---------------------------------------------------------------- STRICT
@@ -259,6 +275,7 @@ template <typename G>
 __global__ void __launch_bounds__(BLOCK)
     k_strict_prepare(active_set_t as, G g, Status want, bool pull,
                      int64_t *d) {
+  stamp_begin(as.dg_work);
   const int64_t N = as.get_size();
   const int64_t *rows = pull ? g.dgr_row_ptr : g.dg_row_ptr;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < N;
@@ -331,6 +348,7 @@ __device__ __forceinline__ int64_t strict_next_owner(const int64_t *s_scan,
 template <class B>
 __global__ void __launch_bounds__(BLOCK)
     k_push_strict(B body, const int64_t *__restrict__ scan) {
+  const unsigned long long t0 = wall_clock64();
   __shared__ int s_stage[B::STAGE_LDS];
   auto st = body.stage(s_stage);
   __shared__ int64_t s_scan[SCHUNK + 1];
@@ -381,7 +399,7 @@ __global__ void __launch_bounds__(BLOCK)
     k0 = nk;
   }
   body.emit_flush(st, s_stage);
-  add_work(body.as.dg_work, ne, 0);
+  add_work(body.as.dg_work, t0, ne, 0);
 }
 
 // ---------------------------------------------------------------- TWC
@@ -395,6 +413,7 @@ __global__ void __launch_bounds__(BLOCK)
   wave_stage_t<CAP> st[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) st[k].buf = s_stage[k][threadIdx.x >> LOG_WAVE];
+  stamp_begin(as.dg_work);
   const int64_t N = as.get_size();
   const int64_t *rows = pull ? g.dgr_row_ptr : g.dg_row_ptr;
   const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -420,6 +439,7 @@ __global__ void __launch_bounds__(BLOCK)
 
 template <class B>
 __global__ void __launch_bounds__(BLOCK) k_push_twc(B body) {
+  const unsigned long long t0 = wall_clock64();
   __shared__ int s_stage[B::STAGE_LDS];
   auto st = body.stage(s_stage);
   const int lane = lane_id();
@@ -494,7 +514,7 @@ __global__ void __launch_bounds__(BLOCK) k_push_twc(B body) {
     }
   }
   body.emit_flush(st, s_stage);
-  add_work(body.as.dg_work, ne, nv);
+  add_work(body.as.dg_work, t0, ne, nv);
 }
 
 }  // namespace gsw

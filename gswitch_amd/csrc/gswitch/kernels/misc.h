@@ -9,11 +9,13 @@
 #include "../data_structures/active_set.h"
 #include "../data_structures/functor.h"
 #include "../utils/wave.h"
+#include "expand_push.h"
 
 namespace gsw {
 
 template <typename G, typename F>
 __global__ void __launch_bounds__(BLOCK) k_expand_ec(active_set_t as, G g, F f) {
+  const unsigned long long t0 = wall_clock64();
   const int64_t N = as.get_size();
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < N;
        idx += (int64_t)gridDim.x * blockDim.x) {
@@ -23,6 +25,7 @@ __global__ void __launch_bounds__(BLOCK) k_expand_ec(active_set_t as, G g, F f) 
     f.update((int)(vv >> 32), (int)(vv & 0xffffffffll),
              (typename G::edge_t *)nullptr);
   }
+  add_work(as.dg_work, t0, 0, 0);
 }
 
 // lab[v] <- lab[lab[v]]; *changed = 1 if any label moved

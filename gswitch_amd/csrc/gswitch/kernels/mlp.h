@@ -160,10 +160,11 @@ __device__ __forceinline__ void block_features(const sel_dev_t &d, float act,
 // STAT_SLOTS slots (lane s reads slot s) into info[0..6), clears the slots
 // for the next pass and, with the learned selector on (d.w set), turns the
 // counters into the 12 features and writes the class the network picks to
-// info[6], which the host reads with the counters. A kernel of its own
+// info[6], which the host reads with the counters; `info` is pinned host
+// memory and info[MARK] = seq tells the host that they are there. A kernel of its own
 // rather than a tail of the pass, so the pass keeps its register budget.
 __global__ void __launch_bounds__(BLOCK)
-    k_stat_finish(sel_dev_t d, long long *slots, long long *info) {
+    k_stat_finish(sel_dev_t d, long long *slots, long long *info, long long seq) {
   static_assert(STAT_SLOTS == WAVE, "one lane per partial slot");
   __shared__ mlp_block_sh_t s;
   __shared__ long long tot[6];
@@ -186,12 +187,18 @@ __global__ void __launch_bounds__(BLOCK)
       }
     }
   }
-  if (!d.w) return;  // uniform over the workgroup
+  if (!d.w) {  // uniform over the workgroup
+    if (threadIdx.x == 0) publish(info + stat_t::MARK, seq);
+    return;
+  }
   __syncthreads();
   block_features(d, (float)tot[0], (float)tot[1], (float)tot[2], (float)tot[3],
                  (float)tot[4], s);
   const int cls = mlp_block_select(d.w, d.mask, s);
-  if (threadIdx.x == 0) info[6] = cls;
+  if (threadIdx.x == 0) {
+    info[6] = cls;
+    publish(info + stat_t::MARK, seq);
+  }
 }
 
 // ---- batch paths (training, tests) -----------------------------------------

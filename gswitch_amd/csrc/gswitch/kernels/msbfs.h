@@ -376,10 +376,11 @@ __global__ void __launch_bounds__(BLOCK)
 }
 
 // End of a level, one workgroup: the slots' sum to `out` (pinned host
-// memory), the slots cleared for the next level.
+// memory), then its mark; the slots cleared for the next level.
 constexpr int MS_COUNTS = 66;  // newly, newly_deg, per_src
+constexpr int MS_MARK = 72;    // (in the padding of a slot)
 __global__ void __launch_bounds__(BLOCK)
-    k_msbfs_finish(ms_counters_t *c, unsigned long long *out) {
+    k_msbfs_finish(ms_counters_t *c, unsigned long long *out, unsigned long long seq) {
   __shared__ unsigned long long sh[BLOCK / WAVE][WAVE + 2];
   static_assert(sizeof(ms_counters_t) % 8 == 0, "slots of whole words");
   constexpr int NW = BLOCK / WAVE, W = sizeof(ms_counters_t) / 8;
@@ -400,7 +401,10 @@ __global__ void __launch_bounds__(BLOCK)
 #pragma unroll
     for (int i = 0; i < NW; ++i) t += sh[i][threadIdx.x];
     out[threadIdx.x] = t;
+    __threadfence_system();
   }
+  __syncthreads();
+  if (threadIdx.x == 0) publish(out + MS_MARK, seq);
 }
 
 __global__ void __launch_bounds__(BLOCK)

@@ -247,6 +247,7 @@ template <class Bd, typename MSG>
 __global__ void __launch_bounds__(PB_BLOCK) k_pb_scatter(Bd body, pb_t pb) {
   constexpr int CAP = PB_LDS_BYTES / (int)sizeof(MSG);
   __shared__ MSG s_msg[CAP];
+  stamp_begin(body.as.dg_work);
   const int32_t *pc = pb.p1 + 4 * (int64_t)blockIdx.x;
   const int c = pc[0], b0 = pc[1], b1 = pc[2];
   if (b0 >= b1) return;  // padding of the XCD-aware piece order
@@ -328,6 +329,7 @@ __global__ void __launch_bounds__(PB_BLOCK) k_pb_scatter(Bd body, pb_t pb) {
 // in atomics.)
 template <class Bd, typename MSG>
 __global__ void __launch_bounds__(PB_BLOCK) k_pb_gather(Bd body, pb_t pb) {
+  const unsigned long long t0 = wall_clock64();
   using WA = typename Bd::WA;
   constexpr int CAP = PB_LDS_BYTES / (int)sizeof(WA);
   __shared__ WA s_acc[CAP];
@@ -454,7 +456,7 @@ __global__ void __launch_bounds__(PB_BLOCK) k_pb_gather(Bd body, pb_t pb) {
         body.f.compAtomic(body.f.wa_of(lo), tot, body.g);
     }
   }
-  add_work<PB_BLOCK>(body.as.dg_work, threadIdx.x == 0 ? (unsigned long long)(e1 - e0) : 0ull,
+  add_work<PB_BLOCK>(body.as.dg_work, t0, threadIdx.x == 0 ? (unsigned long long)(e1 - e0) : 0ull,
                      0ull);
 }
 

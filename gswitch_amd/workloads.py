@@ -46,7 +46,7 @@ def main(argv=None):
     ap.add_argument("--capture", type=int, default=0,
                     help="bfs: device-resident loop, levels per replay")
     ap.add_argument("--no-profile", action="store_true",
-                    help="no per-expand hipEvents (records keep no times)")
+                    help="records keep no per-expand times")
     a = ap.parse_args(argv)
     if a.app == "copy":
         g = gsw.stream_copy(a.mib << 20, a.repeat)

@@ -119,7 +119,7 @@ typedef struct {
   int32_t verbose;    /* per-level log on stderr */
   int32_t twc_small;  /* TWC bins: degree < twc_small -> thread */
   int32_t twc_large;  /*           degree < twc_large -> wavefront */
-  int32_t profile;    /* time every expand with hipEvents */
+  int32_t profile;    /* record every expand's time (device clock) */
   int32_t pull_kernel; /* from-all pulls of unweighted graphs: 0 TWOD as
                           length-binned source slices, STRICT as a merge-path
                           walk; 1 both as segmented reductions; 2 (default)
