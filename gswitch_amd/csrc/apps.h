@@ -351,6 +351,9 @@ int run_vc(engine_t &en, active_set_t &as, G &g, F &f, const run_opts_t &o,
       en.conf.show_hints(std::cerr);
       fprintf(stderr, "\n");
     }
+    // (a training record per level needs the host at every level)
+    if (!o.verbose && record_sink().path.empty())
+      level += en.executor.run_ahead(as, g, f, en.fets, en.conf, o.max_levels - level - 1);
     if (as.finish(g, f, en.conf)) break;
   }
   return level;

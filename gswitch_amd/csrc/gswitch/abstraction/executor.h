@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../data_structures/active_set.h"
+#include "../kernels/ahead.h"
 #include "../kernels/expand_pull.h"
 #include "../kernels/expand_push.h"
 #include "../kernels/filter.h"
@@ -49,16 +50,19 @@ struct executor_t {
   void clear_log() { log.clear(); }
   void release() { clear_log(); }
 
+  void need_clock() {
+    if (clock_khz > 0) return;
+    int dev = 0, khz = 0;
+    H_ERR(hipGetDevice(&dev));
+    H_ERR(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+    GSW_REQUIRE(khz > 0, gsw::E_HIP, "device reports no wall clock rate");
+    clock_khz = khz;
+  }
+
   // Work counters and times of all logged expands (one report).
   void finalize_log(active_set_t &as) {
     if (log.empty() || !as.dg_work_base) return;
-    if (clock_khz == 0) {
-      int dev = 0, khz = 0;
-      H_ERR(hipGetDevice(&dev));
-      H_ERR(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
-      GSW_REQUIRE(khz > 0, gsw::E_HIP, "device reports no wall clock rate");
-      clock_khz = khz;
-    }
+    need_clock();
     const int64_t rows = std::min<int64_t>((int64_t)log.size(), WORK_ROWS);
     const unsigned long long *w = as.read_work(rows);
     for (size_t i = 0; i < log.size(); ++i) {
@@ -256,6 +260,125 @@ struct executor_t {
     fets.last_time = stat.last_time;
     fets.avg_time = stat.avg_time;
     conf.conf_first_round = false;
+  }
+
+  // After a fused expand whose next queue is not empty: further fused levels
+  // without the host (kernels/ahead.h), at most max_levels. Returns how many
+  // ran and leaves the state as the last one's expand() would. The rule
+  // selector's fused WM push only: the learned selector looks at every fused
+  // level's queue length.
+  template <typename G, typename F>
+  int run_ahead(active_set_t &as, G &g, F &f, feature_t &fets, config_t &conf,
+                int64_t max_levels) {
+    using namespace gsw;
+    if (!conf.conf_fuse_inspect || conf.conf_centric != VC || conf.policy_mlp ||
+        conf.verbose || conf.conf_compensation || conf.conf_lb != WM || as.fmt != Queue ||
+        as.queue.mode != Normal || as.converged || as.known_active <= 0)
+      return 0;
+    hipStream_t st = stream();
+    need_clock();
+    queue_t &q = as.queue;
+    const bool prune = conf.conf_pruning;
+    if (!as.dg_ahead) H_ERR(hipMalloc(&as.dg_ahead, sizeof(ahead_t)));
+    if (!as.h_ahead) {
+      H_ERR(hipHostMalloc((void **)&as.h_ahead, sizeof(long long) * (AHEAD_WORDS + 3)));
+      as.h_ahead[AHEAD_WORDS + 2] = 0;
+    }
+    if (!prune && !as.ahead_bits.dg_bits) as.ahead_bits.build(as.size);
+    ahead_t *a = (ahead_t *)as.dg_ahead;
+    long long *h = as.h_ahead, *mark = h + AHEAD_WORDS + 2;
+    const ahead_t *ha = (const ahead_t *)h;
+    uint64_t *const bits[2] = {as.bitmap.visited.dg_bits, as.ahead_bits.dg_bits};
+    const int64_t n_bits = prune ? 0 : as.bitmap.visited.n_words;
+    // the exit rule of expand(), on device times: the host's share of a level
+    // (about 25 us there) counts in its average, hence the allowance
+    const bool rule = fets.pattern == Idem && !conf.force.has_fusion;
+    const double allow = clock_khz * 0.1;
+    double ticks = 0;
+    const int per = BLOCK / (WAVE / conf.wm_vpw);  // frontier vertices per workgroup
+    const double size = (double)as.size;
+    int ran = 0, in_buf = q.cursor ^ 1;  // buffer of the next input
+    bool begin = true, slow = false;
+    long long nq = as.known_active;
+    double growth = (double)nq / (double)MAX(1LL, log.back().frontier);
+    while (nq > 0 && !slow) {
+      int k = (int)MIN((int64_t)AHEAD, max_levels - ran);
+      k = (int)MIN((int64_t)k, (int64_t)WORK_ROWS - 1 - (int64_t)log.size());
+      if (k <= 0) break;
+      // grids for twice the growth seen last; an explosion (a random graph's)
+      // is followed level by level once it reaches a good part of the graph
+      int grids[AHEAD];
+      double est = (double)nq, reach[AHEAD];
+      for (int j = 0; j < k; ++j) {
+        const double up = j == 0 ? est : MIN(size, 2 * est);
+        grids[j] = (int)MAX(1.0, MIN((double)MAX_GRID, std::ceil(up / per)));
+        reach[j] = grids[j] >= MAX_GRID ? 2147483647.0
+                                        : MIN(2147483647.0, MAX(up, 4.0 * grids[j] * per));
+        est = MIN(size, est * MAX(growth, 1.25));
+        if (growth > 2 && est * 32 > size) k = j + 1;
+      }
+      if (begin)
+        hipLaunchKernelGGL(k_ahead_begin, dim3(grid_for(ran == 0 ? n_bits : 1)), dim3(BLOCK),
+                           0, st, a, ran % AHEAD_SLOTS, (int)nq, bits[0], bits[1],
+                           ran == 0 ? n_bits : 0);
+      for (int j = 0; j < k; ++j) {
+        const int i = ran + j;
+        as.select_work_row((int)log.size() + j);
+        active_set_t la = as;
+        la.queue.cursor = in_buf ^ (j & 1);
+        // (output_size() is sizes + (cursor ^ 1): the slot after the input's)
+        la.queue.sizes = a->q + (i + 1) % AHEAD_SLOTS - (la.queue.cursor ^ 1);
+        if (!prune) la.bitmap.visited.dg_bits = bits[i & 1];
+        G gl = g;
+        gl.level = g.level + 1 + j;
+        using Bd = push_body<G, F, true>;
+        hipLaunchKernelGGL(k_push_wm_ahead<Bd>, dim3(grids[j]), dim3(BLOCK), 0, st,
+                           Bd{la, gl, f, conf, prune ? nullptr : bits[(i & 1) ^ 1]},
+                           conf.wm_vpw, a, j, i % AHEAD_SLOTS, (int)reach[j]);
+      }
+      const long long seq = *mark + 1;
+      hipLaunchKernelGGL(k_ahead_end, dim3(1), dim3(64), 0, st, (const ahead_t *)a,
+                         (const int32_t *)as.dg_ctrl, h, mark, seq);
+      H_ERR(hipGetLastError());
+      await_mark(mark, seq, st);
+      GSW_REQUIRE(h[AHEAD_WORDS + 1] == 0, E_OVERFLOW, "frontier queue overflow");
+      begin = false;
+      level_record_t rec = log.back();
+      int done = 0;
+      for (int j = 0; j < k; ++j) {
+        if (ha->sizes[j] == 0) break;
+        if ((double)ha->sizes[j] > reach[j]) {
+          begin = true;  // its length back into the slot
+          break;
+        }
+        rec.level = ++g.level;
+        rec.frontier = rec.active = ha->sizes[j];
+        rec.inactive = as.known_inactive;
+        log.push_back(rec);
+        ++done;
+        const double dt =
+            (double)((j + 1 < k ? ha->clock[j + 1] : h[AHEAD_WORDS]) - ha->clock[j]);
+        if (rule && ran + done > 1 && dt > 5 * (ticks / (ran + done - 1)) + allow) slow = true;
+        ticks += dt;
+      }
+      nq = done < k ? ha->sizes[done] : ha->q[(ran + k) % AHEAD_SLOTS];
+      if (done > 0) growth = (double)nq / (double)log.back().frontier;
+      ran += done;
+      in_buf ^= done & 1;
+    }
+    if (ran == 0) return 0;
+    // as after expand(): the cursor on the consumed queue, the next one's
+    // length behind it
+    q.cursor = in_buf ^ 1;
+    set_one_async<int32_t>(q.sizes + in_buf, (int)nq);
+    q.host_sizes[in_buf] = (int)nq;
+    as.known_active = nq;
+    if (nq == 0) as.halt_host();
+    if (slow && nq > 0) {
+      conf.conf_fuse_inspect = false;
+      as.swap_queues();
+    }
+    return ran;
   }
 
   template <typename G, typename F>

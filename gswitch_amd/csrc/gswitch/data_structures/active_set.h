@@ -166,6 +166,11 @@ struct active_set_t {
   int work_rows = 0;                          // rows written since their last clear
   unsigned long long *h_work = nullptr;       // pinned: folded rows, then a mark
   int64_t h_work_rows = 0;
+  // fused levels run ahead of the host (kernels/ahead.h): their device state
+  // and the second de-duplication bitmap, on first use
+  void *dg_ahead = nullptr;
+  long long *h_ahead = nullptr;  // pinned: the device words, then a mark
+  bits_t ahead_bits;
   // host-side counts of the current frontier (from the inspector's
   // counters, or the root): the filter sizes its output queue with them
   // without a device round trip
@@ -200,6 +205,11 @@ struct active_set_t {
     if (h_work) hipHostFree(h_work);
     h_work = nullptr;
     h_work_rows = 0;
+    if (dg_ahead) hipFree(dg_ahead);
+    if (h_ahead) hipHostFree(h_ahead);
+    h_ahead = nullptr;
+    if (ahead_bits.dg_bits) ahead_bits.release();
+    dg_ahead = nullptr;
     dg_ctrl = nullptr;
     dg_work = dg_work_base = nullptr;
     dg_block_count = nullptr;

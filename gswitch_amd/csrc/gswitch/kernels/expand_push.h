@@ -81,9 +81,17 @@ template <typename G, typename F, bool FUSED> struct push_body {
   G g;
   F f;
   config_t conf;
+  // run-ahead levels that de-duplicate within the level: the bitmap that
+  // marked this level's queue (its set bits are the queue's vertices), cleared
+  // by their consumers for the level after
+  uint64_t *clear_bits = nullptr;
 
   __device__ __forceinline__ const int64_t *rows() const { return g.dg_row_ptr; }
   __device__ __forceinline__ const int32_t *cols() const { return g.dg_adj_list; }
+  __device__ __forceinline__ void taken(int v) const {
+    if constexpr (FUSED)
+      if (clear_bits) clear_bits[v >> 6] = 0;
+  }
 
   // true when u must be appended to the next queue (fused only)
   __device__ __forceinline__ bool operator()(int v, int u, int64_t e) {
@@ -167,11 +175,11 @@ __global__ void __launch_bounds__(BLOCK) k_push_tm(B body) {
 }
 
 // ---------------------------------------------------------------- WM
-template <class B>
 // A wavefront takes `vpw` frontier items (64, 32, 16 or 8) and walks their
 // edges 64 at a time: with a small mean degree fewer items per wavefront
 // means more wavefronts in flight and fewer dependent 64-edge steps each.
-__global__ void __launch_bounds__(BLOCK) k_push_wm(B body, int vpw) {
+template <class B>
+__device__ __forceinline__ void push_wm_range(B &body, int vpw, int64_t N) {
   const unsigned long long t0 = wall_clock64();
   __shared__ int s_stage[B::STAGE_LDS];
   auto st = body.stage(s_stage);
@@ -180,7 +188,6 @@ __global__ void __launch_bounds__(BLOCK) k_push_wm(B body, int vpw) {
   __shared__ int64_t s_start[BLOCK];
   const int lane = lane_id();
   const int off = threadIdx.x & ~(WAVE - 1);
-  const int64_t N = body.as.get_size();
   const Status want = body.conf.want();
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> LOG_WAVE;
   const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> LOG_WAVE;
@@ -191,6 +198,7 @@ __global__ void __launch_bounds__(BLOCK) k_push_wm(B body, int vpw) {
     int64_t start = 0;
     int deg = 0;
     if (v >= 0) {
+      body.taken(v);
       start = body.rows()[v];
       deg = (int)(body.rows()[v + 1] - start);
       ++nv;
@@ -218,6 +226,10 @@ __global__ void __launch_bounds__(BLOCK) k_push_wm(B body, int vpw) {
   }
   body.emit_flush(st, s_stage);
   add_work(body.as.dg_work, t0, ne, nv);
+}
+template <class B>
+__global__ void __launch_bounds__(BLOCK) k_push_wm(B body, int vpw) {
+  push_wm_range(body, vpw, body.as.get_size());
 }
 
 // ---------------------------------------------------------------- CM
