@@ -23,6 +23,7 @@
 #include "../kernels/filter.h"
 #include "../kernels/misc.h"
 #include "../kernels/pb.h"
+#include "../kernels/pull_rows.h"
 #include "../kernels/twod.h"
 #include "config.h"
 #include "features.h"
@@ -417,7 +418,19 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
     using MSG = typename pb_msg<F>::type;
     using WAt = typename F::wa_t;
     const bool use_pb = lb == TWOD && conf.pb_pull && g.pb;
-    if (use_pb) {
+    // a small graph whose every vertex stays active: whole rows, the filter
+    // with them (kernels/pull_rows.h), unless the blocked layout is asked for
+    bool use_rows = false;
+    if constexpr (pb_has_filter_acc<F>::value)
+      use_rows = use_pb && conf.counts_known && conf.wa_zero &&
+                 g.nedges <= rows_max_edges() && !std::getenv("GSW_PB_ECAP") &&
+                 !std::getenv("GSW_PB_GROUPS");
+    if (use_rows) {
+      rows_ensure(*g.rowbins, g.dgr_row_ptr, g.nvertexs);
+      if (!f.data.dg_ra2)
+        H_ERR(hipMalloc((void **)&f.data.dg_ra2,
+                        sizeof(typename F::ra_t) * (g.nvertexs + 1)));
+    } else if (use_pb) {
       pb_ensure(g, PB_LDS_BYTES / (int)sizeof(MSG), PB_LDS_BYTES / (int)sizeof(WAt));
       pb_vals(*g.pb, sizeof(MSG));
     } else if (lb == TWOD) {
@@ -521,6 +534,23 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
                              dim3(BLOCK), 0, st, body);
           break;
         case TWOD: {
+          if constexpr (pb_has_filter_acc<F>::value) {
+            if (use_rows) {
+              const rowbins_t &rb = *g.rowbins;
+              int4 first;
+              first.x = rows_blocks(rb, 3);
+              first.y = first.x + rows_blocks(rb, 2);
+              first.z = first.y + rows_blocks(rb, 1);
+              first.w = first.z + rows_blocks(rb, 0);
+              F out = f;
+              std::swap(out.data.dg_ra, out.data.dg_ra2);
+              hipLaunchKernelGGL((k_pull_rows<Bd, F>), dim3(first.w), dim3(BLOCK), 0, st,
+                                 body, out, rb, first);
+              std::swap(f.data.dg_ra, f.data.dg_ra2);
+              conf.filter_done = true;
+              break;
+            }
+          }
           if (use_pb) {
             // propagation blocking: messages to slots, then slots to targets
             // group by group (consecutive bins): a group's phase 2 follows

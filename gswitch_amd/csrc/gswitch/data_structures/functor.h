@@ -40,8 +40,10 @@ template <typename WA, typename RA> struct vdata_t {
       hipFree(dg_ra);
       free(h_ra);
     }
+    if (dg_ra2) hipFree(dg_ra2);
     dg_wa = nullptr;
     dg_ra = nullptr;
+    dg_ra2 = nullptr;
     h_wa = nullptr;
     h_ra = nullptr;
   }
@@ -72,6 +74,7 @@ template <typename WA, typename RA> struct vdata_t {
   WA zero{};
   WA *dg_wa = nullptr;
   RA *dg_ra = nullptr;
+  RA *dg_ra2 = nullptr;  // the other of two read attributes (on first use)
   WA *h_wa = nullptr;  // host mirrors (plain arrays: the functor is copied
   RA *h_ra = nullptr;  // byte-wise into every kernel)
   int64_t size = 0;

@@ -150,6 +150,12 @@ struct pb_t {
   }
 };
 
+// Targets listed by in-degree class (kernels/pull_rows.h, on first use).
+struct rowbins_t {
+  int32_t *list = nullptr;  // [n], class k from off[k] on
+  int64_t off[4] = {0, 0, 0, 0}, cnt[4] = {0, 0, 0, 0};
+};
+
 template <GraphFmt fmt, typename E> struct device_graph_t {};
 
 template <typename E> struct device_graph_t<CSR, E> {
@@ -185,6 +191,7 @@ template <typename E> struct device_graph_t<CSR, E> {
   // host-side handle of the propagation-blocked layout (kernels/pb.h), owned
   // the same way
   pb_t *pb = nullptr;
+  rowbins_t *rowbins = nullptr;  // likewise
 
   // Upload a host CSR. `w` is converted to E when E is not Empty.
   int64_t build(const gsw_host::HostGraph &hg) {
@@ -194,6 +201,7 @@ template <typename E> struct device_graph_t<CSR, E> {
     level = 0;
     twod = new twod_t();
     pb = new pb_t();
+    rowbins = new rowbins_t();
     int64_t bytes = 0;
     H_ERR(hipMalloc((void **)&dg_row_ptr, sizeof(int64_t) * (nvertexs + 1)));
     H_ERR(hipMemcpy(dg_row_ptr, hg.row_ptr.data(),
@@ -259,6 +267,9 @@ template <typename E> struct device_graph_t<CSR, E> {
       pb->release();
       delete pb;
       pb = nullptr;
+      if (rowbins->list) hipFree(rowbins->list);
+      delete rowbins;
+      rowbins = nullptr;
     }
     if (directed) {
       hipFree(dgr_row_ptr);

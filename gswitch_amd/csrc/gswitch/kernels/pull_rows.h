@@ -1,0 +1,159 @@
+// From-all pull of a small graph in one launch per level, the functor's
+// filter included.
+//
+// Where the sources' state fits the L2, gathering it per edge is cheaper than
+// propagation blocking's two passes over per-edge messages, whose pieces also
+// leave most of the chip idle on a small graph. Targets are listed once per
+// graph by in-degree: a lane takes a row of up to 8 edges, eight lanes one of
+// up to 128, a wavefront one of up to 2048, a workgroup a longer one, so that
+// every row is summed in one place and the rank update can follow at once. The
+// update writes the other of two source-state arrays (the messages of the same
+// level still read the first), which then change places.
+// Latency bounds it: a list entry, row offsets, columns and messages are a
+// chain of four loads.
+// Measured per PageRank iteration, against propagation blocking: R-MAT 11 (26 K
+// edges) 28.8 -> 6.8 us, R-MAT 14 (228 K) 35.6 -> 7.8, a web graph of 728 K
+// edges 20.9 -> 8.4, R-MAT 18 (7.6 M) 57 -> 36; but 16.4 M edges over 2 M
+// sources 82 -> 129 and R-MAT 20 (31 M) 103 -> 179, hence the limit.
+#pragma once
+#include "expand_pull.h"
+#include "pb.h"
+
+namespace gsw {
+
+constexpr int ROWS_CLASSES = 4;
+constexpr int ROWS_LANE = 8, ROWS_GROUP = 128, ROWS_WAVE = 2048;  // longest row of a class
+constexpr int64_t ROWS_MAX_EDGES = 8 << 20;
+
+// (GSW_ROWS_EDGES: another limit, for sweeps)
+inline int64_t rows_max_edges() {
+  const char *e = std::getenv("GSW_ROWS_EDGES");
+  return e ? std::atoll(e) : ROWS_MAX_EDGES;
+}
+
+__device__ __forceinline__ int rows_class(int64_t deg) {
+  return deg <= ROWS_LANE ? 0 : deg <= ROWS_GROUP ? 1 : deg <= ROWS_WAVE ? 2 : 3;
+}
+
+// pass 0: class sizes into cnt[0..4); pass 1: rows into list, class k from
+// cnt[k] on (the offsets, moved along)
+__global__ void __launch_bounds__(BLOCK)
+    k_rows_list(const int64_t *__restrict__ rows, int64_t n, int32_t *list,
+                unsigned long long *cnt) {
+  const int lane = lane_id();
+  const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> LOG_WAVE;
+  const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> LOG_WAVE;
+  for (int64_t base = wave << 6; base < n; base += nwaves << 6) {
+    const int64_t v = base + lane;
+    const int c = v < n ? rows_class(rows[v + 1] - rows[v]) : -1;
+#pragma unroll
+    for (int k = 0; k < ROWS_CLASSES; ++k) {
+      const uint64_t m = ballot(c == k);
+      if (!m) continue;
+      unsigned long long at = 0;
+      if (lane == 0) at = atomicAdd(cnt + k, (unsigned long long)__popcll(m));
+      at = __shfl(at, 0, 64);
+      if (list && c == k) list[at + rank_below(m)] = (int32_t)v;
+    }
+  }
+}
+
+inline void rows_ensure(rowbins_t &rb, const int64_t *rows, int64_t n) {
+  if (rb.list) return;
+  unsigned long long *cnt = nullptr, h[ROWS_CLASSES];
+  int32_t *list = nullptr;
+  H_ERR(hipMalloc((void **)&cnt, sizeof(h)));
+  try {
+    H_ERR(hipMalloc((void **)&list, sizeof(int32_t) * (n + 1)));
+    const dim3 grid(grid_for((n + 63) / 64 * 64));
+    fill_async<unsigned long long>(cnt, 0ull, ROWS_CLASSES);
+    hipLaunchKernelGGL(k_rows_list, grid, dim3(BLOCK), 0, stream(), rows, n,
+                       (int32_t *)nullptr, cnt);
+    H_ERR(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, stream()));
+    sync();
+    unsigned long long off[ROWS_CLASSES], at = 0;
+    for (int k = 0; k < ROWS_CLASSES; ++k) {
+      off[k] = at;
+      rb.off[k] = (int64_t)at;
+      rb.cnt[k] = (int64_t)h[k];
+      at += h[k];
+    }
+    GSW_REQUIRE((int64_t)at == n, E_INTERNAL_CHECK, "row classes miss rows");
+    H_ERR(hipMemcpyAsync(cnt, off, sizeof(off), hipMemcpyHostToDevice, stream()));
+    hipLaunchKernelGGL(k_rows_list, grid, dim3(BLOCK), 0, stream(), rows, n, list, cnt);
+    H_ERR(hipGetLastError());
+    sync();
+  } catch (...) {
+    (void)hipFree(cnt);
+    (void)hipFree(list);
+    throw;
+  }
+  H_ERR(hipFree(cnt));
+  rb.list = list;
+}
+
+// workgroups of each class
+inline int rows_blocks(const rowbins_t &rb, int k) {
+  const int per[ROWS_CLASSES] = {BLOCK, BLOCK / 8, BLOCK / WAVE, 1};
+  return (int)((rb.cnt[k] + per[k] - 1) / per[k]);
+}
+
+// the messages of in-edges [s, e) of one row, lane `i` of `w`
+template <class Bd>
+__device__ __forceinline__ typename Bd::WA rows_sum(Bd &body, int64_t s, int64_t e, int i,
+                                                    int w) {
+  typename Bd::WA acc{};
+  for (int64_t j = s + i; j < e; j += 4 * w) {
+    int u[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u[r] = j + r * w < e ? body.cols()[j + r * w] : -1;
+    typename Bd::WA m[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) m[r] = body.msg(u[r] >= 0 ? u[r] : u[0], 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (u[r] >= 0) body.f.comp(&acc, m[r], body.g);
+  }
+  return acc;
+}
+
+// `out`: the functor whose filter writes the other source-state array.
+template <class Bd, class F>
+__global__ void __launch_bounds__(BLOCK)
+    k_pull_rows(Bd body, F out, rowbins_t rb, int4 first_block) {
+  const unsigned long long t0 = wall_clock64();
+  using WA = typename Bd::WA;
+  __shared__ WA s_part[BLOCK / WAVE];
+  const int b = blockIdx.x, t = threadIdx.x;
+  // longest rows first: first_block holds the first workgroup of classes 2, 1, 0
+  const int k = b < first_block.x ? 3 : b < first_block.y ? 2 : b < first_block.z ? 1 : 0;
+  const int bk = b - (k == 3 ? 0 : k == 2 ? first_block.x : k == 1 ? first_block.y : first_block.z);
+  const int w = k == 0 ? 1 : k == 1 ? 8 : k == 2 ? WAVE : BLOCK;  // threads per row
+  const int64_t i = (int64_t)bk * (BLOCK / w) + t / w;
+  const bool ok = i < rb.cnt[k];
+  int v = 0;
+  int64_t s = 0, e = 0;
+  if (ok) {
+    v = rb.list[rb.off[k] + i];
+    s = body.rows()[v];
+    e = body.rows()[v + 1];
+  }
+  WA acc = rows_sum(body, s, e, t % w, w);
+  for (int o = MIN(w, WAVE) >> 1; o > 0; o >>= 1) {
+    const WA x = shfl_xor_any(acc, o);
+    body.f.comp(&acc, x, body.g);
+  }
+  if (k == 3) {  // uniform over the workgroup
+    if (lane_id() == 0) s_part[t >> LOG_WAVE] = acc;
+    __syncthreads();
+    acc = s_part[0];
+    for (int j = 1; j < BLOCK / WAVE; ++j) body.f.comp(&acc, s_part[j], body.g);
+  }
+  if (ok && t % w == 0) {
+    *out.ra_of(v) = *body.f.ra_of(v);
+    (void)out.filter_acc(v, acc, body.g);
+  }
+  add_work(body.as.dg_work, t0, ok && t % w == 0 ? (unsigned long long)(e - s) : 0ull, 0ull);
+}
+
+}  // namespace gsw

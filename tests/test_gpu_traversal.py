@@ -251,6 +251,43 @@ def test_pagerank(gsw, orc, gset, variant, pull_kernel):
         assert max_rel(pr, ref) <= PR_TOL, (variant, gname, max_rel(pr, ref))
 
 
+@pytest.mark.parametrize("directed", [False, True])
+def test_pagerank_whole_rows(gsw, orc, monkeypatch, directed):
+    """The whole-row pull of small graphs: rows of 0, 1, 8, 9, 128, 129, 2048,
+    2049 and 5000 in-edges (the edges of its classes), odd and even iteration
+    counts (its two rank arrays change places), a second damping on the same
+    graph, and the same ranks as the blocked layout gives."""
+    rng = np.random.default_rng(5)
+    degs = [1, 8, 9, 128, 129, 2048, 2049, 5000, 3, 64]
+    n = 6007
+    src = np.concatenate([rng.choice(n - 20, d, replace=False) + 10 for d in degs])
+    dst = np.concatenate([np.full(d, k) for k, d in enumerate(degs)])
+    h = gsw.from_edges(n, src, dst, directed=directed)
+    g = gsw.Graph(h)
+    def oracle(damping, iters):
+        if not directed:
+            return orc.pagerank(h.row_ptr, h.col, damping, iters)
+        out = np.maximum(np.diff(h.row_ptr), 1)
+        s = np.repeat(np.arange(n), np.diff(h.row_ptr))
+        r = np.full(n, 1 - damping)
+        for _ in range(iters):
+            r = (1 - damping) + damping * np.bincount(h.col, (r / out)[s], n)
+        return r
+
+    for damping, iters in [(0.85, 1), (0.85, 2), (0.85, 7), (0.5, 4), (0.85, 0)]:
+        ranks = {}
+        for limit in ("8388608", "0"):
+            monkeypatch.setenv("GSW_ROWS_EDGES", limit)
+            ranks[limit] = g.pagerank(damping, iters, configs="Pull-Bitmap-TWOD-Standalone")
+            assert max_rel(ranks[limit], oracle(damping, iters)) <= PR_TOL
+            recs = g.records()
+            assert len(recs) == iters
+            assert all(r["edges"] == g.m and r["kernel"] == 2 for r in recs)
+        # sums in 64 bits, ranks in 32: one rounding apart at most per iteration
+        assert max_rel(ranks["0"], ranks["8388608"].astype(float)) <= 2 ** -23 * max(iters, 1)
+    g.close()
+
+
 @pytest.mark.parametrize("slice_kb", [1, 4, 64])
 def test_pagerank_twod_slices(gsw, orc, monkeypatch, slice_kb):
     """TWOD with several source slices (one launch each): R-MAT 12 has
