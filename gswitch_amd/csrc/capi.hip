@@ -1749,10 +1749,8 @@ gsw_status gsw_bc(gsw_graph *G, int32_t root, const gsw_run_opts *opts,
                        dim3(gsw::BLOCK), 0, st, c.f.data.dg_wa, h.data.dg_wa,
                        h.data.dg_ra, n, G->d_flag);
     H_ERR(hipGetLastError());
-    H_ERR(hipMemcpyAsync(G->h_flag, G->d_flag, sizeof(int32_t),
-                         hipMemcpyDeviceToHost, st));
-    gsw::sync();
-    const int deepest = G->h_flag[0];
+    c.as.report(G->d_flag, 1, nullptr, 0);
+    const int deepest = c.as.h_ctrl[0];
     prepare_engine(c, o, !opts || opts->profile);
     fets.centric = VC;
     fets.pattern = ASSO;

@@ -44,6 +44,7 @@ struct config_t {
   bool conf_fuse_inspect = false;
   bool conf_lite = false;
   bool conf_window = false;
+  double work_hint = 0;  // edges of the level where the inspector counted them
   int wm_vpw = 64;  // frontier items per wavefront of the WM push
   // TM pulls take each target's first in-edge from the per-vertex copy
   bool pull_first = false;

@@ -14,6 +14,7 @@
 // queue's length, which also tells convergence). Queue lengths are otherwise
 // known on the host from the inspector's counts.
 #pragma once
+#include <cmath>
 #include <vector>
 
 #include "../data_structures/active_set.h"
@@ -150,13 +151,18 @@ struct executor_t {
                                : as.known_active + as.known_inactive;
     GSW_REQUIRE(expect <= (q.mode == Normal ? q.capacity : q.capacity - q.offset_out),
                 gsw::E_OVERFLOW, "frontier does not fit the queue");
-    gsw::set_one_async<int32_t>(out_size, 0);
+    const bool normal = q.mode == Normal;
+    if (!normal || !q.slot_zero[out_slot]) gsw::set_one_async<int32_t>(out_size, 0);
+    if (normal) q.slot_zero[out_slot] = false;
     if (!conf.conf_sorted) {
+      const int wpw = gsw::filter_wpw(nw);
+      // (the consumed length is left alone where it is known to be zero)
+      int32_t *consumed = normal && !q.slot_zero[q.cursor] ? q.sizes + q.cursor : nullptr;
       hipLaunchKernelGGL(gsw::k_filter_unsorted,
-                         dim3(gsw::grid_for((nw + gsw::FILTER_WPT - 1) / gsw::FILTER_WPT,
-                                            gsw::BLOCK, 1024)),
-                         dim3(gsw::BLOCK), 0, gsw::stream(), as, target, n, out,
-                         out_size);
+                         dim3(gsw::grid_for((nw + wpw - 1) / wpw, gsw::BLOCK / gsw::WAVE, 1024)),
+                         dim3(gsw::BLOCK), 0, gsw::stream(), as, target, n, wpw, out,
+                         out_size, consumed);
+      q.consumed_clear = consumed != nullptr;
     } else {
       const int nb = (int)MAX(1, MIN(1024, (nw + gsw::BLOCK - 1) / gsw::BLOCK));
       const int64_t wpb = (nw + nb - 1) / nb;
@@ -211,6 +217,16 @@ struct executor_t {
       // in-neighbour is a hub, far more walks end there)
       conf.pull_first = conf.conf_pruning && fets.push_workload_ratio >= 0.1;
     }
+    // (a queue of the active vertices, or of the inactive ones)
+    conf.work_hint = 0;
+    if (!conf.conf_fuse_inspect && as.fmt == Queue) {
+      if (conf.conf_dir == Push && conf.conf_target == Active)
+        conf.work_hint = fets.push_workload;
+      else if (conf.conf_dir == Pull && conf.conf_target == Inactive)
+        conf.work_hint = fets.pull_workload;
+    }
+    if (conf.conf_fuse_inspect && as.queue.mode == Normal)
+      as.queue.slot_zero[as.queue.cursor ^ 1] = false;
     dispatch(as, g, f, conf, stat);
     log.push_back(rec);
     if (conf.verbose) {
@@ -371,6 +387,7 @@ struct executor_t {
     // as after expand(): the cursor on the consumed queue, the next one's
     // length behind it
     q.cursor = in_buf ^ 1;
+    q.slot_zero[0] = q.slot_zero[1] = false;
     set_one_async<int32_t>(q.sizes + in_buf, (int)nq);
     q.host_sizes[in_buf] = (int)nq;
     as.known_active = nq;
@@ -390,6 +407,32 @@ struct executor_t {
 inline int expand_grid(int64_t N, int per) {
   int64_t g = (N + per - 1) / per;
   return (int)MAX(1, MIN((int64_t)gsw::MAX_GRID, g));
+}
+
+// slot prefix of a queue frontier of N items into the STRICT workset
+template <typename G>
+void strict_scan(active_set_t &as, G &g, const config_t &conf, int64_t N, bool pull) {
+  using namespace gsw;
+  const int64_t nb = (N + SCAN_TILE - 1) / SCAN_TILE;
+  if (nb <= SCAN_OWN_TILES) {
+    hipLaunchKernelGGL(k_strict_prepare_sums<G>, dim3((unsigned)nb), dim3(BLOCK), 0, stream(),
+                       as, g, conf.conf_target, pull, as.workset.dg_scan, as.workset.dg_bsum);
+    hipLaunchKernelGGL(k_scan_tile_apply_own, dim3((unsigned)nb), dim3(BLOCK), 0, stream(),
+                       as.workset.dg_scan, N, (const int64_t *)as.workset.dg_bsum);
+    return;
+  }
+  hipLaunchKernelGGL(k_strict_prepare<G>, dim3(grid_for(N)), dim3(BLOCK), 0, stream(), as, g,
+                     conf.conf_target, pull, as.workset.dg_scan);
+  scan_exclusive_inplace(as.workset.dg_scan, N, as.workset.dg_bsum);
+}
+
+// STRICT workgroups share the slots evenly: no more of them than 256-slot
+// shares where the inspector counted the level's edges (a level of 3 K edges:
+// 12 workgroups instead of 2048 that each search for an empty share)
+inline int strict_grid(const config_t &conf, int64_t N) {
+  if (conf.work_hint <= 0) return gsw::MAX_GRID;
+  const double slots = conf.work_hint + (double)N;
+  return (int)MAX(1.0, MIN((double)gsw::MAX_GRID, std::ceil(slots / gsw::BLOCK)));
 }
 
 template <typename G, typename F>
@@ -474,13 +517,10 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
           default: {  // STRICT
             const int64_t *scan = nullptr;  // bitmap: implicit rows[v] + v
             if (as.fmt == Queue) {
-              hipLaunchKernelGGL(k_strict_prepare<G>, dim3(grid_for(N)),
-                                 dim3(BLOCK), 0, st, as, g, conf.conf_target,
-                                 false, as.workset.dg_scan);
-              scan_exclusive_inplace(as.workset.dg_scan, N, as.workset.dg_bsum);
+              strict_scan(as, g, conf, N, false);
               scan = as.workset.dg_scan;
             }
-            hipLaunchKernelGGL(k_push_strict<Bd>, dim3(MAX_GRID), dim3(BLOCK),
+            hipLaunchKernelGGL(k_push_strict<Bd>, dim3(strict_grid(conf, N)), dim3(BLOCK),
                                0, st, body, scan);
             break;
           }
@@ -609,13 +649,10 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
             break;
           }
           if (as.fmt == Queue) {
-            hipLaunchKernelGGL(k_strict_prepare<G>, dim3(grid_for(N)),
-                               dim3(BLOCK), 0, st, as, g, conf.conf_target,
-                               true, as.workset.dg_scan);
-            scan_exclusive_inplace(as.workset.dg_scan, N, as.workset.dg_bsum);
+            strict_scan(as, g, conf, N, true);
             scan = as.workset.dg_scan;
           }
-          hipLaunchKernelGGL(k_pull_strict<Bd>, dim3(MAX_GRID), dim3(BLOCK), 0,
+          hipLaunchKernelGGL(k_pull_strict<Bd>, dim3(strict_grid(conf, N)), dim3(BLOCK), 0,
                              st, body, scan);
           break;
         }

@@ -224,6 +224,8 @@ struct active_set_t {
     if (queue.mode == Normal) {
       nq = queue.max_levels + 2;
       queue.host_sizes[0] = queue.host_sizes[1] = 0;
+      queue.slot_zero[0] = queue.slot_zero[1] = true;
+      queue.consumed_clear = false;
     }
     if (!traceback) {
       queue.cursor = 0;
@@ -384,7 +386,10 @@ struct active_set_t {
   // (queue_t::swap, src/data_structures/queue.cuh:113-127).
   void swap_queues() {
     if (queue.mode == Normal) {
-      gsw::set_one_async<int32_t>(queue.sizes + queue.cursor, 0);
+      if (!queue.consumed_clear && !queue.slot_zero[queue.cursor])
+        gsw::set_one_async<int32_t>(queue.sizes + queue.cursor, 0);
+      queue.consumed_clear = false;
+      queue.slot_zero[queue.cursor] = true;
       queue.host_sizes[queue.cursor] = 0;
       queue.cursor ^= 1;
     } else if (queue.traceback) {

@@ -83,6 +83,11 @@ struct queue_t {
     st.flush_block(output_size(), output_base(), output_capacity(), overflow, s_cnt);
   }
 
+  // host knowledge of Normal mode's device lengths: a slot that holds zero,
+  // and that the latest filter cleared the consumed one
+  bool slot_zero[2] = {false, false};
+  bool consumed_clear = false;
+
   // ---- host side (a plain array: queue_t is copied byte-wise to kernels) --
   int *host_sizes = nullptr;  // sizes known on the host, per slot
 };

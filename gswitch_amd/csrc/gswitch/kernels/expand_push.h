@@ -96,8 +96,13 @@ template <typename G, typename F, bool FUSED> struct push_body {
   // true when u must be appended to the next queue (fused only)
   __device__ __forceinline__ bool operator()(int v, int u, int64_t e) {
     if constexpr (!FUSED) {
+      // A level-synchronous functor that prunes by visits is idempotent (BFS):
+      // it writes the same value whichever edge comes first, so its standalone
+      // levels store it without a mark (15 K edges into 4096 vertices: with
+      // the atomics on 64 words the launch took 44 us, without 9).
       bool go = true;
-      if (conf.conf_pruning) go = as.bitmap.mark_duplicate_lite(u);
+      if (conf.conf_pruning && !is_level_sync<F>::value)
+        go = as.bitmap.mark_duplicate_lite(u);
       if (go && !conf.conf_toall) go = as.bitmap.is_inactive(u);
       if (go) {
         auto msg = f.emit(v, g.fetch_edata(e), g);
@@ -295,6 +300,35 @@ __global__ void __launch_bounds__(BLOCK)
     const int v = as.fetch(i, want);
     d[i] = 1 + ((v >= 0) ? (rows[v + 1] - rows[v]) : 0);
   }
+}
+
+// The same with the sum of every scan tile (one workgroup each), for
+// frontiers that k_scan_tile_apply_own scans.
+template <typename G>
+__global__ void __launch_bounds__(BLOCK)
+    k_strict_prepare_sums(active_set_t as, G g, Status want, bool pull, int64_t *d,
+                          int64_t *bsum) {
+  __shared__ int64_t sh[BLOCK / WAVE];
+  stamp_begin(as.dg_work);
+  const int64_t N = as.get_size();
+  const int64_t *rows = pull ? g.dgr_row_ptr : g.dg_row_ptr;
+  const int64_t lo = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x;
+  // the items' loads together: a queue entry, then its two row offsets
+  int v[SCAN_ITEMS];
+  int64_t x[SCAN_ITEMS], s = 0;
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k)
+    v[k] = lo + k * BLOCK < N ? as.fetch(lo + k * BLOCK, want) : -1;
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k) x[k] = v[k] >= 0 ? rows[v[k] + 1] - rows[v[k]] : 0;
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k)
+    if (lo + k * BLOCK < N) {
+      d[lo + k * BLOCK] = x[k] + 1;
+      s += x[k] + 1;
+    }
+  s = block_sum(s, sh);
+  if (threadIdx.x == 0) bsum[blockIdx.x] = s;
 }
 
 // Slot prefix of the STRICT partition: an explicit int64 scan of (deg + 1)

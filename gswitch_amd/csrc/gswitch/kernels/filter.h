@@ -4,8 +4,8 @@
 // __filter_unfixed, src/kernel_libs/filter.cuh:30-112) walks byte words with
 // a 32-lane scan and one atomic per warp, giving a queue sorted only inside
 // each warp's stripe. Here:
-//  * unsorted: each lane owns one 64-bit word; a DPP wave scan of popcounts
-//    and one atomicAdd per wavefront reserve the output range;
+//  * unsorted: each lane owns one 64-bit word; a workgroup scan of popcounts
+//    and one atomicAdd per workgroup reserve the output range;
 //  * sorted:   workgroups own contiguous word ranges; pass 1 counts per
 //    workgroup, pass 2 offsets each workgroup by the counts before it and
 //    writes ids in ascending order, so the queue is globally sorted.
@@ -37,36 +37,46 @@ __device__ __forceinline__ void write_word_ids(uint64_t m, int64_t w,
   }
 }
 
-// Each thread owns FILTER_WPT consecutive words; a workgroup scan of their
-// popcounts and one atomicAdd per workgroup step reserve the output range
-// (one atomic per 64 Ki vertices: a counter shared by every wavefront of
-// the grid serialises its atomics).
-constexpr int FILTER_WPT = 4;
+// A wavefront takes `wpw` consecutive words (one lane each), a workgroup scan
+// of their popcounts and one atomicAdd per workgroup step reserve the output
+// range (a counter shared by every wavefront of the grid serialises its
+// atomics), and the wavefront writes word after word, lane b the id of bit b:
+// coalesced, and a dense word costs one store. `wpw` shares the words out over
+// 512 wavefronts (2048: the 512 atomics alone took 6 us) before a wavefront
+// takes the most it can, 64. (With four words per thread and a thread writing
+// their ids one by one, 160 K ids of a 262 K-vertex bitmap took 25 us.)
+// *consumed (not null): the length of the queue that the last level read,
+// cleared here for its next use as an output.
+inline int filter_wpw(int64_t nw) {
+  return (int)MAX((int64_t)1, MIN((int64_t)WAVE, (nw + 511) / 512));
+}
 __global__ void __launch_bounds__(BLOCK)
-    k_filter_unsorted(active_set_t as, Status target, int64_t n,
-                      int32_t *out, int32_t *out_size) {
+    k_filter_unsorted(active_set_t as, Status target, int64_t n, int wpw,
+                      int32_t *out, int32_t *out_size, int32_t *consumed) {
   __shared__ int sh[BLOCK / WAVE];
   __shared__ int s_base;
+  if (consumed && blockIdx.x == 0 && threadIdx.x == 0) *consumed = 0;
+  const int lane = lane_id();
+  const int wv = threadIdx.x >> LOG_WAVE;
+  constexpr int NW = BLOCK / WAVE;
   const int64_t nw = (n + 63) >> 6;
-  const int64_t step = (int64_t)gridDim.x * BLOCK * FILTER_WPT;
-  for (int64_t w0 = (int64_t)blockIdx.x * BLOCK * FILTER_WPT; w0 < nw; w0 += step) {
-    const int64_t w = w0 + (int64_t)threadIdx.x * FILTER_WPT;
-    uint64_t m[FILTER_WPT];
-    int c = 0;
-#pragma unroll
-    for (int k = 0; k < FILTER_WPT; ++k) {
-      m[k] = (w + k < nw) ? target_word(as, w + k, target, n) : 0ull;
-      c += __popcll(m[k]);
-    }
+  const int64_t step = (int64_t)gridDim.x * NW * wpw;
+  for (int64_t b0 = (int64_t)blockIdx.x * NW * wpw; b0 < nw; b0 += step) {
+    const int64_t w0 = b0 + (int64_t)wv * wpw, w = w0 + lane;
+    const uint64_t m = lane < wpw && w < nw ? target_word(as, w, target, n) : 0ull;
     int tot;
-    int pos = block_exclusive_scan(c, tot, sh);
+    const int pos = block_exclusive_scan(__popcll(m), tot, sh);
     if (threadIdx.x == 0) s_base = tot ? atomicAdd(out_size, tot) : 0;
     __syncthreads();
-    pos += s_base;
-#pragma unroll
-    for (int k = 0; k < FILTER_WPT; ++k) {
-      write_word_ids(m[k], w + k, out, pos);
-      pos += __popcll(m[k]);
+    const int base = s_base + pos;
+    uint64_t some = ballot(m != 0ull);
+    while (some) {
+      const int j = __builtin_ctzll(some);
+      some &= some - 1;
+      const uint64_t bits = ((uint64_t)(uint32_t)readlane((int)(m >> 32), j) << 32) |
+                            (uint32_t)readlane((int)(uint32_t)m, j);
+      const int at = readlane(base, j);
+      if ((bits >> lane) & 1ull) out[at + rank_below(bits)] = (int32_t)(((w0 + j) << 6) + lane);
     }
     __syncthreads();  // s_base and sh are reused by the next step
   }

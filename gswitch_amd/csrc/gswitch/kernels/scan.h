@@ -107,6 +107,40 @@ __global__ void __launch_bounds__(BLOCK)
   }
 }
 
+// k_scan_tile_apply with the tile's offset summed up by its own workgroup
+// (nb <= SCAN_OWN_TILES tile sums), and the total behind the last item: one
+// launch instead of two.
+constexpr int SCAN_OWN_TILES = 1024;
+__global__ void __launch_bounds__(BLOCK)
+    k_scan_tile_apply_own(int64_t *__restrict__ a, int64_t N,
+                          const int64_t *__restrict__ bsum) {
+  __shared__ int64_t sh[BLOCK / WAVE + 1];
+  __shared__ int64_t s_before;
+  int64_t before = 0;
+  for (int i = threadIdx.x; i < (int)blockIdx.x; i += BLOCK) before += bsum[i];
+  before = block_sum(before, sh);
+  if (threadIdx.x == 0) s_before = before;
+  __syncthreads();
+  const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
+  int64_t x[SCAN_ITEMS];
+  int64_t s = 0;
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k) {
+    const int64_t i = base + k;
+    x[k] = (i < N) ? a[i] : 0;
+    s += x[k];
+  }
+  int64_t total;
+  int64_t run = block_exclusive_scan_any(s, total, sh) + s_before;
+#pragma unroll
+  for (int k = 0; k < SCAN_ITEMS; ++k) {
+    const int64_t i = base + k;
+    if (i < N) a[i] = run;
+    run += x[k];
+  }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) a[N] = s_before + total;
+}
+
 // Host driver. `bsum` must hold ceil(N / 2048) + 1 entries.
 inline void scan_exclusive_inplace(int64_t *a, int64_t N, int64_t *bsum) {
   const int64_t nb64 = (N + SCAN_TILE - 1) / SCAN_TILE;

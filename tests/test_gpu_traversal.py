@@ -172,6 +172,30 @@ def test_sssp_requires_weights(gsw, gset):
         g.sssp(0)
 
 
+@pytest.mark.parametrize("width", [1, 63, 64, 65, 2047, 2048, 2049, 4097, 40000, 300000])
+def test_queue_frontiers_at_tile_edges(gsw, orc, width):
+    """Queue frontiers of every size around a bitmap word and a scan tile,
+    dense and sparse words, through the filter and the STRICT prefix: a root,
+    `width` children, one grandchild each."""
+    kids = 1 + np.arange(width)
+    src = np.concatenate([np.zeros(width, int), kids])
+    dst = np.concatenate([kids, kids + width])
+    rng = np.random.default_rng(width)
+    for shuffle in (False, True):
+        perm = rng.permutation(2 * width + 1) if shuffle else np.arange(2 * width + 1)
+        h = gsw.from_edges(2 * width + 1, perm[src], perm[dst],
+                           rng.integers(1, 65, len(src)).astype(np.uint32))
+        g = gsw.Graph(h)
+        root = int(perm[0])
+        ref, dist = orc.bfs(h.row_ptr, h.col, root), orc.spfa(h.row_ptr, h.col, h.w, root)
+        for lb in ("STRICT", "WM"):
+            for fmt in ("Queue", "SortedQueue"):
+                cfg = "Push-%s-%s-Standalone" % (fmt, lb)
+                assert np.array_equal(g.bfs(root, configs=cfg), ref), cfg
+                assert np.array_equal(g.sssp(root, configs=cfg), dist), cfg
+        g.close()
+
+
 # ---------------------------------------------------------------- CC
 @pytest.mark.parametrize("gname", ["rmat12", "grid", "er", "ba"])
 @pytest.mark.parametrize("variant", [None, "x-Queue-x-x", "x-Bitmap-x-x"])
