@@ -915,15 +915,12 @@ gsw::dobfs_t do_view(gsw_graph *G) {
   d.ctrl = G->do_ctrl;
   d.hist = G->do_hist;
   // switching thresholds and the heavy-vertex degree (defaults measured on
-  // MI355X; the variables exist for sweeps). A vertex is heavy from 256 edges
-  // on (one wavefront needs about 2.5 us per 64 of them: the root of R-MAT 22
-  // with 3039 edges took 121 us below a fixed 4096), and on large graphs from
-  // so many that a top-down frontier, which holds fewer than m / alpha edges,
-  // cannot overflow the list.
-  const double heavy = MIN(4096.0, MAX(256.0, std::ceil((double)G->hg.m / (14.0 * DO_HCAP))));
+  // MI355X; the variables exist for sweeps). A root is heavy from 256 edges on
+  // (one wavefront needs about 2.5 us per 64 of them).
   d.alpha = (float)env_num("GSW_DO_ALPHA", 14.0);
   d.beta = (float)env_num("GSW_DO_BETA", 24.0);
-  d.heavy_deg = (int)env_num("GSW_DO_HEAVY", heavy);
+  d.heavy_deg = (int)env_num("GSW_DO_HEAVY", 4096.0);
+  d.root_heavy = MIN(256, d.heavy_deg);
   // a wavefront scans 64 degrees of at most heavy_deg each in int32
   GSW_REQUIRE(d.alpha > 0 && d.beta > 0 && d.heavy_deg >= 64 &&
                   d.heavy_deg <= INT32_MAX / WAVE,

@@ -41,8 +41,10 @@
 // Dependent loads bound both: with 64 words per wavefront whatever their
 // number, vertices taken word by word, and one in-edge probed at a time, BFS
 // over 300 random graphs (2.5 M vertices, 38.9 M edges) spent 2.8 ms in
-// k_do_expand, now 0.56 ms; R-MAT 22 0.44, now 0.27 ms (with heavy vertices
-// from 560 edges on instead of 4096).
+// k_do_expand, now 0.56 ms; R-MAT 22 0.44, now 0.27 ms (its root
+// of 3039 edges split over the grid as well: a root is heavy from 256 edges on.
+// A lower bound for found vertices costs more than it saves: each is an atomic
+// on the list's length, R-MAT 24 from its largest hub 0.42 -> 0.61 ms at 2271).
 //
 // The result is the BFS level array, the same whatever the directions.
 #pragma once
@@ -98,13 +100,14 @@ struct dobfs_t {
   long long *ctrl = nullptr;       // [DO_TOTAL]
   long long *hist = nullptr;       // [DO_HIST][DO_HIST_W] per-level history
                                    // (pinned host memory)
-  int heavy_deg = 4096;
+  int heavy_deg = 4096;            // of a found vertex
+  int root_heavy = 256;            // of a root (level 0)
   float alpha = 14.f, beta = 24.f;
 };
 
 // Query reset: levels -1 (root 0), visited and frontier words zero except
 // the root's bit, control block for level 0 (top-down from the root; the
-// root is the heavy list of level 0 when its degree is above heavy_deg).
+// root is the heavy list of level 0 when its degree is above root_heavy).
 // root < 0: every vertex unreached and every word zero; the roots are then
 // set by k_do_seed.
 __global__ void __launch_bounds__(BLOCK) k_do_reset(dobfs_t d, int root) {
@@ -128,7 +131,7 @@ __global__ void __launch_bounds__(BLOCK) k_do_reset(dobfs_t d, int root) {
       d.ctrl[DO_NF] = 1;
       d.ctrl[DO_MF] = deg;
       d.ctrl[DO_VISE] = deg;
-      if (deg > d.heavy_deg) {
+      if (deg > d.root_heavy) {
         d.heavy[0] = root;
         d.hpre[0] = 0;
         d.hpre[1] = deg;
@@ -141,7 +144,7 @@ __global__ void __launch_bounds__(BLOCK) k_do_reset(dobfs_t d, int root) {
 
 // Several roots (distinct ids, after k_do_reset with root < 0): level 0,
 // their bits in the visited and level-0 frontier words, and the level's
-// counters. Roots of more than heavy_deg edges are not listed: the heavy
+// counters. Roots of more than root_heavy edges are not listed: the heavy
 // list is marked overflowed, so each is walked by its own wavefront.
 __global__ void __launch_bounds__(BLOCK)
     k_do_seed(dobfs_t d, const int32_t *__restrict__ roots, int64_t k) {
@@ -158,7 +161,7 @@ __global__ void __launch_bounds__(BLOCK)
     const int deg = d.odeg[r];
     ++nf;
     mf += deg;
-    heavy |= deg > d.heavy_deg;
+    heavy |= deg > d.root_heavy;
   }
   const long long a = block_sum(nf, sh);
   const long long c = block_sum(mf, sh);
@@ -285,6 +288,7 @@ __global__ void __launch_bounds__(BLOCK) k_do_expand(dobfs_t d) {
 
   if (!pull) {
     const bool hovf = ctrl[DO_HOVF] != 0;
+    const int heavy_deg = t.L == 0 ? d.root_heavy : d.heavy_deg;
     // listed heavy vertices: their edges split evenly over the grid
     const int64_t HE = hovf ? 0 : ctrl[DO_HE];
     if (HE > 0) {
@@ -327,7 +331,7 @@ __global__ void __launch_bounds__(BLOCK) k_do_expand(dobfs_t d) {
           const int o = owner_search(&s_pre[off], WAVE, i);
           v = (int)(((w0 + o) << 6) + select_bit(s_word[off + o], i - s_pre[off + o]));
           deg = d.odeg[v];
-          if (deg > d.heavy_deg) {
+          if (deg > heavy_deg) {
             alone = hovf;  // walked below by this wavefront
             deg = 0;       // otherwise walked by the heavy pass
           } else {

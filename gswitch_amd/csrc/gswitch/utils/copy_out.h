@@ -66,16 +66,20 @@ __global__ void __launch_bounds__(BLOCK)
   }
 }
 
-// A pinned ring (two halves of OUT_HALF bytes) and its marks.
+// A pinned ring of `cap` bytes, at most two halves of OUT_HALF (smaller where
+// only small results were asked for: pinning takes time by the page), and its
+// marks.
 struct out_ring_t {
   int dev = -1;
+  size_t cap = 0;
   char *buf = nullptr;
   uint32_t *marks = nullptr;
   uint32_t seq = 0;  // of the last launch
-  void build(int d) {
+  void build(int d, size_t bytes) {
     dev = d;
+    cap = bytes;
     const size_t mb = sizeof(uint32_t) * 2 * OUT_PIECES * OUT_MARK;
-    H_ERR(hipHostMalloc((void **)&buf, 2 * OUT_HALF));
+    H_ERR(hipHostMalloc((void **)&buf, cap));
     H_ERR(hipHostMalloc((void **)&marks, mb));
     std::memset(marks, 0, mb);
   }
@@ -97,20 +101,31 @@ struct out_pool_t {
   std::vector<out_ring_t> idle;
   int64_t handles = 0;
 
-  out_ring_t take(int dev) {
+  // a ring of at least `need` bytes; an idle one that is too small goes
+  out_ring_t take(int dev, size_t need) {
+    out_ring_t small;
     {
       std::lock_guard<std::mutex> lock(mu);
       for (size_t i = 0; i < idle.size(); ++i)
         if (idle[i].dev == dev) {
           const out_ring_t r = idle[i];
+          if (r.cap < need && small.buf) continue;
           idle[i] = idle.back();
           idle.pop_back();
-          return r;
+          if (r.cap >= need) {
+            if (small.buf) idle.push_back(small);
+            return r;
+          }
+          small = r;
+          --i;
         }
     }
+    small.release();
     out_ring_t r;
+    size_t cap = 2 * OUT_PIECE;
+    while (cap < need) cap *= 2;
     try {
-      r.build(dev);
+      r.build(dev, cap);
     } catch (...) {
       r.release();
       throw;
@@ -162,13 +177,16 @@ struct out_t {
 };
 
 class copy_out_t {
-  // at most OUT_HALF bytes of one array: one launch into half (index & 1)
+  // at most OUT_HALF bytes of one array: one launch, into a place of its own
+  // in the ring where everything fits, else into half (index & 1)
   struct part_t {
     char *dst;
     const char *src;
     size_t bytes;
     size_t first;  // its first piece
+    size_t slot;   // its first piece's place in the ring
   };
+  bool packed = false;
   std::vector<part_t> parts;
   size_t n_pieces = 0;
   std::vector<std::atomic<size_t>> left;  // pieces of a part not copied on yet
@@ -183,16 +201,16 @@ class copy_out_t {
 
   static size_t pieces_of(size_t bytes) { return (bytes + OUT_PIECE - 1) / OUT_PIECE; }
 
-  // part k, once part k - 2 (the same half) is copied on; called by one
-  // thread at a time, in order
+  // part k, once its place in the ring is free; called by one thread at a
+  // time, in order
   void launch(size_t k) {
     const part_t &q = parts[k];
     if (++ring.seq == 0) ring.seq = 1;
     seqs[k] = ring.seq;
     const int grid = (int)std::min<size_t>(OUT_GRID, pieces_of(q.bytes));
     hipLaunchKernelGGL(k_copy_out, dim3(grid), dim3(BLOCK), 0, st, q.src,
-                       ring.buf + (k & 1) * OUT_HALF, (int64_t)q.bytes,
-                       ring.marks + (k & 1) * OUT_PIECES * OUT_MARK, ring.seq);
+                       ring.buf + q.slot * OUT_PIECE, (int64_t)q.bytes,
+                       ring.marks + q.slot * OUT_MARK, ring.seq);
     H_ERR(hipGetLastError());
     launched.store(k + 1, std::memory_order_release);
   }
@@ -205,7 +223,7 @@ class copy_out_t {
       if (failed) return false;
       pause();
     }
-    const uint32_t *mark = ring.marks + ((k & 1) * OUT_PIECES + i) * OUT_MARK;
+    const uint32_t *mark = ring.marks + (parts[k].slot + i) * OUT_MARK;
     for (int64_t spin = 1; __atomic_load_n(mark, __ATOMIC_ACQUIRE) != seqs[k]; ++spin) {
       if (failed) return false;
       pause();
@@ -232,7 +250,7 @@ class copy_out_t {
         const size_t at = i - parts[k].first;
         if (!await(k, at)) return;
         const size_t b = at * OUT_PIECE;
-        std::memcpy(parts[k].dst + b, ring.buf + (k & 1) * OUT_HALF + b,
+        std::memcpy(parts[k].dst + b, ring.buf + parts[k].slot * OUT_PIECE + b,
                     std::min(OUT_PIECE, parts[k].bytes - b));
         // the worker that empties a half refills it (parts are emptied in
         // order: part k + 1 is launched, its predecessor's half is this one)
@@ -251,7 +269,7 @@ class copy_out_t {
   // launch every part whose half is free (under mu)
   void refill() {
     for (size_t k = launched; k < parts.size(); ++k) {
-      if (k >= 2 && left[k - 2].load(std::memory_order_acquire) != 0) return;
+      if (!packed && k >= 2 && left[k - 2].load(std::memory_order_acquire) != 0) return;
       launch(k);
     }
   }
@@ -276,7 +294,7 @@ class copy_out_t {
       total += o.bytes;
       for (size_t b = 0; b < o.bytes; b += OUT_HALF) {
         const size_t len = std::min(OUT_HALF, o.bytes - b);
-        parts.push_back({(char *)o.dst + b, (const char *)o.src + b, len, n_pieces});
+        parts.push_back({(char *)o.dst + b, (const char *)o.src + b, len, n_pieces, 0});
         n_pieces += pieces_of(len);
       }
     }
@@ -284,7 +302,10 @@ class copy_out_t {
     left = std::vector<std::atomic<size_t>>(parts.size());
     for (size_t k = 0; k < parts.size(); ++k) left[k] = pieces_of(parts[k].bytes);
     seqs.resize(parts.size());
-    ring = out_pool().take(dev);
+    packed = n_pieces <= 2 * OUT_PIECES;
+    for (size_t k = 0; k < parts.size(); ++k)
+      parts[k].slot = packed ? parts[k].first : (k & 1) * OUT_PIECES;
+    ring = out_pool().take(dev, packed ? n_pieces * OUT_PIECE : 2 * OUT_HALF);
     std::vector<std::thread> th;
     try {
       std::lock_guard<std::mutex> lock(mu);

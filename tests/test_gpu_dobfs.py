@@ -227,3 +227,35 @@ def test_device_bfs_bottom_up_probe_remainders(gsw, orc):
     left = (ref == -1) & (indeg > 0)
     assert recs[1]["edges"] == int(indeg[reached2 | left].sum())
     g.close()
+
+
+@pytest.mark.parametrize("leaves", [255, 256, 257, 4096, 4097, 9000])
+def test_device_bfs_heavy_roots(gsw, orc, leaves):
+    """Roots around the heavy root's degree, alone (split over the grid) and
+    with others (walked by their own wavefront), and found vertices of the
+    same degree one level down."""
+    n = 2 * leaves + 3
+    src = np.concatenate([np.zeros(leaves, int), [1], np.full(leaves, leaves + 1)])
+    dst = np.concatenate([1 + np.arange(leaves), [leaves + 1], leaves + 2 + np.arange(leaves)])
+    h = gsw.from_edges(n, src, dst)
+    g = gsw.Graph(h)
+    for alpha in (1e-9, 14):
+        with env(GSW_DO_ALPHA=alpha):
+            for root in (0, leaves + 1, n - 2):
+                ref = orc.bfs(h.row_ptr, h.col, root)
+                assert np.array_equal(g.bfs(root, capture=4), ref)
+                recs = g.records()
+                assert recs[0]["dir"] == "Push"
+                for L, r in enumerate(recs):
+                    if r["dir"] == "Push":  # heavy vertices are expanded once
+                        at = ref == L
+                        assert r["verts"] == int(at.sum())
+                        assert r["edges"] == int(np.diff(h.row_ptr)[at].sum())
+            off = np.array([0, leaves + 1, n], np.int64)
+            lv, _ = g.batch_bfs_cc(off)
+            a = orc.bfs(h.row_ptr, h.col, 0)
+            b = orc.bfs(h.row_ptr, h.col, leaves + 1)
+            far = np.iinfo(np.int32).max
+            want = np.minimum(np.where(a < 0, far, a), np.where(b < 0, far, b))
+            assert np.array_equal(lv, np.where(want == far, -1, want))
+    g.close()
