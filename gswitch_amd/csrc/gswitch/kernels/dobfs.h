@@ -43,8 +43,16 @@
 // over 300 random graphs (2.5 M vertices, 38.9 M edges) spent 2.8 ms in
 // k_do_expand, now 0.56 ms; R-MAT 22 0.44, now 0.27 ms (its root
 // of 3039 edges split over the grid as well: a root is heavy from 256 edges on.
-// A lower bound for found vertices costs more than it saves: each is an atomic
-// on the list's length, R-MAT 24 from its largest hub 0.42 -> 0.61 ms at 2271).
+// The lower bound is for roots only: a found heavy vertex is an atomic on the
+// list's length (R-MAT 24 from its largest hub: 0.61 ms at 2271, 0.58 at 4096).
+//
+// Not every root gains. From the largest hub, whose search is bottom-up from
+// level 1 on, the version with whole words per wavefront was faster: R-MAT 24
+// 0.42 against 0.58 ms now, R-MAT 22 0.165 against 0.19 (R-MAT 20: 0.21 against
+// 0.13). From a low-degree root R-MAT 24 went 0.92 -> 0.79, R-MAT 22 0.67 -> 0.38.
+// On R-MAT 24 every large level is slower, the first push included (45 -> 83 us,
+// then 165 -> 246, 71 -> 108, 31 -> 51); occupancy is the same 8 waves per SIMD and 1, 2 or
+// 4 probes at a time make no difference (0.58-0.60 ms).
 //
 // The result is the BFS level array, the same whatever the directions.
 #pragma once
