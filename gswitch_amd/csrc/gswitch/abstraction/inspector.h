@@ -78,12 +78,13 @@ struct inspector_t {
       need = false;
     }
     if (need && conf.counts_known) {
-      // (the filter pass is skipped when the last expand applied it)
+      // (the filter pass is skipped when the last expand applied it; it counts
+      // nothing, since no finish kernel would clear the slots after it)
       if (!conf.filter_done) {
         hipLaunchKernelGGL((gsw::k_inspect_vc<device_graph_t<CSR, E>, F>),
                            dim3(gsw::grid_for((g.nvertexs + 63) / 64 * 64)),
                            dim3(gsw::BLOCK), 0, gsw::stream(), as, g, f,
-                           stat.slots());
+                           (long long *)nullptr);
         H_ERR(hipGetLastError());
       }
       conf.filter_done = false;

@@ -14,7 +14,8 @@
 // one-workgroup finish kernel (k_stat_finish) sums the slots into
 // `h_runtime_info` (pinned host memory: six counters, the learned class and a
 // mark that the host polls for) and clears them, so the slots are zero
-// between passes.
+// between passes and from run to run: every launch that adds into them is
+// followed by a finish kernel.
 #pragma once
 #include "../model/class_tree.h"
 #include "../model/mlp.h"

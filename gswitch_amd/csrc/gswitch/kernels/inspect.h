@@ -31,6 +31,8 @@ __device__ __forceinline__ void flush_max(T x, T *sh, long long *slot) {
   if (threadIdx.x == 0 && r) atomicMax((long long *)slot, (long long)r);
 }
 
+// `slots` null: the bitmaps only. Counts in the slots stay there until
+// k_stat_finish takes them, so a pass that none follows must leave them alone.
 template <typename G, typename F>
 __global__ void __launch_bounds__(BLOCK)
     k_inspect_vc(active_set_t as, G g, F f, long long *slots) {
@@ -67,6 +69,7 @@ __global__ void __launch_bounds__(BLOCK)
       as.bitmap.inactive.dg_bits[w] = nm;
     }
   }
+  if (!slots) return;  // uniform
   long long *slot = stat_slot(slots);
   flush_sum(act, sh, slot + 0);
   flush_sum(inact, sh, slot + 1);

@@ -312,6 +312,33 @@ def test_pagerank_whole_rows(gsw, orc, monkeypatch, directed):
     g.close()
 
 
+@pytest.mark.parametrize("first", [dict(configs="Pull-Queue-WM-Standalone"),
+                                   dict(configs="Push-Bitmap-STRICT-Standalone"),
+                                   dict(pull_kernel=0), dict(pull_kernel=1)])
+@pytest.mark.parametrize("eps", [1e9, 1e-3])
+def test_pagerank_eps_after_fixed_iterations(gsw, gset, first, eps):
+    """A run that counts active vertices after runs on the same handle whose
+    inspections count none: same ranks and levels as on a fresh handle (eps =
+    1e9 ends at the first inspection)."""
+    h, _ = gset["rmat12"]
+    g = gsw.Graph(h)
+    for iters in (1, 4):
+        g.pagerank(0.85, iters, **first)
+        for configs in ("Pull-Queue-WM-Standalone", "Pull-Bitmap-WM-Standalone",
+                        "Pull-Bitmap-TWOD-Standalone"):
+            got = g.pagerank(0.85, 60, eps=eps, configs=configs)
+            levels = g.last_stats.levels
+            fresh = gsw.Graph(h)
+            want = fresh.pagerank(0.85, 60, eps=eps, configs=configs)
+            assert levels == fresh.last_stats.levels
+            fresh.close()
+            # 64-bit sums, perhaps in another order: at most a rounding of the
+            # 32-bit ranks apart per level (and errors pass 1e-3 by far more)
+            assert max_rel(got, want.astype(float)) <= 2 ** -23 * max(levels, 1)
+            g.pagerank(0.85, iters, **first)
+    g.close()
+
+
 @pytest.mark.parametrize("slice_kb", [1, 4, 64])
 def test_pagerank_twod_slices(gsw, orc, monkeypatch, slice_kb):
     """TWOD with several source slices (one launch each): R-MAT 12 has
