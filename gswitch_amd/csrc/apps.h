@@ -324,12 +324,14 @@ inline void apply_opts(config_t &conf, const run_opts_t &o) {
   conf.pb_pull = o.pb_pull;
 }
 
-// Generic vertex-centric level loop (application/bfs.cu:87-98 shape).
-// `stop_after_inspect(level)` lets PageRank end on a fold pass. `g` keeps
-// the level the loop ended on (BC's backward pass starts from it).
-template <typename G, typename F, typename Stop>
+// Generic vertex-centric level loop (application/bfs.cu:87-98 shape), at most
+// o.max_levels levels. `stop_after_inspect`: a level cap whose last level is
+// still inspected, which lets PageRank end on a fold pass. `g` keeps the level
+// the loop ended on (BC's backward pass starts from it).
+template <typename G, typename F>
 int run_vc(engine_t &en, active_set_t &as, G &g, F &f, const run_opts_t &o,
-           Stop stop_after_inspect) {
+           int stop_after_inspect = INT_MAX) {
+  const int last = MIN(o.max_levels, stop_after_inspect);
   int level = 0;
   for (level = 0; level < o.max_levels; ++level) {
     as.window_moved = false;
@@ -339,7 +341,7 @@ int run_vc(engine_t &en, active_set_t &as, G &g, F &f, const run_opts_t &o,
     // than expand an empty frontier (a fused choice for it would let the
     // next finish() absorb the new window's updates unexpanded)
     if (as.take_window_moved()) continue;
-    if (stop_after_inspect(level)) break;
+    if (level >= stop_after_inspect) break;
     en.selector.select(en.stats, en.fets, en.conf);
     en.executor.filter(as, g, f, en.stats, en.fets, en.conf);
     g.update_level();
@@ -353,7 +355,7 @@ int run_vc(engine_t &en, active_set_t &as, G &g, F &f, const run_opts_t &o,
     }
     // (a training record per level needs the host at every level)
     if (!o.verbose && record_sink().path.empty())
-      level += en.executor.run_ahead(as, g, f, en.fets, en.conf, o.max_levels - level - 1);
+      level += en.executor.run_ahead(as, g, f, en.fets, en.conf, last - level - 1);
     if (as.finish(g, f, en.conf)) break;
   }
   return level;

@@ -599,7 +599,7 @@ int bfs_engine_run(gsw_graph *G, const gsw_run_opts *opts, int32_t root,
     c.as.init(root, true);
   init_bfs_levels(G, c.f.data.dg_wa, root, d_roots, k);
   GU g = G->dg;
-  const int levels = run_vc(c.en, c.as, g, c.f, o, [](int) { return false; });
+  const int levels = run_vc(c.en, c.as, g, c.f, o);
   H_ERR(hipEventRecord(G->ev1, gsw::stream()));
   return levels;
 }
@@ -1736,7 +1736,7 @@ gsw_status gsw_bc(gsw_graph *G, int32_t root, const gsw_run_opts *opts,
     hipLaunchKernelGGL(k_init_bc, dim3(gsw::grid_for(n)), dim3(gsw::BLOCK), 0, st,
                        c.f.data.dg_wa, n, root);
     GU g = G->dg;
-    int levels = run_vc(c.en, c.as, g, c.f, o, [](int) { return false; });
+    int levels = run_vc(c.en, c.as, g, c.f, o);
     collect_records(G, c.en.executor, c.as);
     std::vector<gsw_level_record> fwd_records = G->records;
 
@@ -1819,7 +1819,7 @@ gsw_status gsw_sssp(gsw_graph *G, int32_t root, const gsw_run_opts *opts,
                        dim3(gsw::BLOCK), 0, st, c.f.data.dg_wa, c.f.data.dg_ra,
                        G->hg.n, root);
     GW g = G->dgw;
-    int levels = run_vc(c.en, c.as, g, c.f, o, [](int) { return false; });
+    int levels = run_vc(c.en, c.as, g, c.f, o);
     H_ERR(hipEventRecord(G->ev1, st));
     const double ms = elapsed(G);
     collect_records(G, c.en.executor, c.as);
@@ -1965,9 +1965,7 @@ gsw_status gsw_pagerank(gsw_graph *G, float damping, int32_t iters, float eps,
                        0, st, c.f.data.dg_wa, c.f.data.dg_ra, G->dg.dg_row_ptr,
                        G->hg.n, damping);
     GU g = G->dg;
-    const int cap = iters;
-    int levels = run_vc(c.en, c.as, g, c.f, o,
-                        [cap](int level) { return level >= cap; });
+    int levels = run_vc(c.en, c.as, g, c.f, o, iters);
     hipLaunchKernelGGL(k_pr_output, dim3(gsw::grid_for(G->hg.n)),
                        dim3(gsw::BLOCK), 0, st, c.f.data.dg_ra,
                        G->dg.dg_row_ptr, G->hg.n, G->d_out_f);
@@ -2028,9 +2026,7 @@ gsw_status gsw_delta_pagerank(gsw_graph *G, float damping, double eps,
                        0, st, c.f.data.dg_wa, c.f.data.dg_ra, G->dg.dg_row_ptr,
                        G->hg.n, damping);
     GU g = G->dg;
-    const int cap = max_iters;
-    const int levels = run_vc(c.en, c.as, g, c.f, o,
-                              [cap](int level) { return level >= cap; });
+    const int levels = run_vc(c.en, c.as, g, c.f, o, max_iters);
     hipLaunchKernelGGL(k_dpr_output, dim3(gsw::grid_for(G->hg.n)), dim3(gsw::BLOCK),
                        0, st, c.f.data.dg_ra, G->hg.n, G->d_out_f);
     H_ERR(hipEventRecord(G->ev1, st));
@@ -2082,7 +2078,7 @@ gsw_status gsw_gc(gsw_graph *G, const gsw_run_opts *opts, int32_t *colors_out,
     gsw::fill_async<int32_t>(c.f.data.dg_wa, -1, G->hg.n);
     gsw::fill_async<int32_t>(c.f.data.dg_ra, -1, G->hg.n);
     GU g = G->dg;
-    const int levels = run_vc(c.en, c.as, g, c.f, o, [](int) { return false; });
+    const int levels = run_vc(c.en, c.as, g, c.f, o);
     H_ERR(hipEventRecord(G->ev1, st));
     const double ms = elapsed(G);
     collect_records(G, c.en.executor, c.as);

@@ -113,3 +113,17 @@ def test_sssp_and_bc_deduplicate_per_level(gsw, orc, spec, configs):
         dep[root] = edep[root] = 0  # (the root is not between any pair)
         assert np.allclose(dep, edep, rtol=1e-10, atol=1e-12)
     g.close()
+
+
+@pytest.mark.parametrize("iters", [0, 1, 2, 3, 9, 20])
+def test_pagerank_iterations_bound_fused_levels(gsw, iters):
+    """Fused PageRank levels keep every vertex queued, so only the iteration
+    count ends them."""
+    h = gsw.rmat(10, 8, seed=4)
+    g = gsw.Graph(h)
+    g.pagerank(0.85, iters, configs=FUSED)
+    assert g.last_stats.levels == iters
+    recs = g.records()
+    assert [r["level"] for r in recs] == list(range(1, iters + 1))
+    assert all(r["edges"] == h.m for r in recs)
+    g.close()
