@@ -44,15 +44,14 @@
 // k_do_expand, now 0.56 ms; R-MAT 22 0.44, now 0.27 ms (its root
 // of 3039 edges split over the grid as well: a root is heavy from 256 edges on.
 // The lower bound is for roots only: a found heavy vertex is an atomic on the
-// list's length (R-MAT 24 from its largest hub: 0.61 ms at 2271, 0.58 at 4096).
+// list's length).
 //
-// Not every root gains. From the largest hub, whose search is bottom-up from
-// level 1 on, the version with whole words per wavefront was faster: R-MAT 24
-// 0.42 against 0.58 ms now, R-MAT 22 0.165 against 0.19 (R-MAT 20: 0.21 against
-// 0.13). From a low-degree root R-MAT 24 went 0.92 -> 0.79, R-MAT 22 0.67 -> 0.38.
-// On R-MAT 24 every large level is slower, the first push included (45 -> 83 us,
-// then 165 -> 246, 71 -> 108, 31 -> 51); occupancy is the same 8 waves per SIMD and 1, 2 or
-// 4 probes at a time make no difference (0.58-0.60 ms).
+// Roots of R-MAT graphs, whole search on the device, against the version with
+// whole words per wavefront: from the largest hub (bottom-up from level 1 on)
+// R-MAT 20 205 -> 125 us, R-MAT 22 164 -> 151, R-MAT 24 416 -> 389; from a root
+// of 144 to 699 edges 909 -> 289, 674 -> 356 and 918 -> 684. One 64-edge step
+// at a time instead of DO_TD = 2 is as fast from the hubs and 6 % slower from
+// the small roots.
 //
 // The result is the BFS level array, the same whatever the directions.
 #pragma once
@@ -269,7 +268,10 @@ __device__ __forceinline__ int select_bit(uint64_t x, int r) {
   return pos;
 }
 
-__global__ void __launch_bounds__(BLOCK) k_do_expand(dobfs_t d) {
+// (8 waves per SIMD asked for: without it the kernel takes 92 SGPRs, of which
+// only 7 waves fit, and the last eighth of the grid runs in a second round.
+// R-MAT 24 from its largest hub 581 -> 389 us, R-MAT 22 189 -> 151.)
+__global__ void __launch_bounds__(BLOCK, 8) k_do_expand(dobfs_t d) {
   __shared__ int s_scan[BLOCK];
   __shared__ int s_pre[BLOCK];
   __shared__ uint64_t s_word[BLOCK];
