@@ -387,7 +387,7 @@ __device__ __forceinline__ void pull_strict_range(B &body, const slots_t sl,
                                                   const int32_t *tgt, int64_t N,
                                                   int64_t bi, int64_t nb,
                                                   bool allow_whole) {
-  const unsigned long long t0 = wall_clock64();
+  stamp_begin(body.as.dg_work);
   using WA = typename B::WA;
   __shared__ int64_t s_scan[SCHUNK + 1];
   __shared__ int64_t s_start[SCHUNK + 1];
@@ -462,7 +462,7 @@ __device__ __forceinline__ void pull_strict_range(B &body, const slots_t sl,
     __syncthreads();
     k0 = nk;
   }
-  add_work(body.as.dg_work, t0, ne, 0);
+  add_work(body.as.dg_work, NO_STAMP, ne, 0);
 }
 
 // ------------------------------------------------- merge-path from-all pull

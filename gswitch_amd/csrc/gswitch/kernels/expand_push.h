@@ -36,13 +36,18 @@ namespace gsw {
 // WORK_ROWS rows apart, so each has a cache line of its own: atomics from
 // every workgroup onto one line serialise on MI355X). Every thread of the
 // workgroup calls it; a workgroup that leaves early leaves as a whole and
-// counts nothing. `t0`: the device clock when the kernel began. (Stamps
-// instead of an event before and after every expand: an event pair costs the
-// stream 7 us, a third of a small PageRank iteration.)
+// counts nothing. `t0`: the device clock when the kernel began, or NO_STAMP
+// where stamp_begin() has told the begin already. (Stamps instead of an event
+// before and after every expand: an event pair costs the stream 7 us, a third
+// of a small PageRank iteration.)
+constexpr unsigned long long NO_STAMP = ~0ull;
 __device__ __forceinline__ unsigned long long *work_slot(unsigned long long *work) {
   return work + (int64_t)(blockIdx.x & (WORK_SLOTS - 1)) * WORK_SLOT_STRIDE;
 }
-// the begin of an expand of several launches, in its first one
+// The begin of an expand of several launches, in its first one; also of a
+// kernel that keeping t0 to its end costs a wave (segmented pulls of BC: 97
+// SGPRs instead of 95; likewise the blocked gather, which takes 58 VGPRs
+// without t0 and 69 with it).
 __device__ __forceinline__ void stamp_begin(unsigned long long *work) {
   if (blockIdx.x == 0 && threadIdx.x == 0)
     atomicMax(work + WORK_BEGIN, ~(unsigned long long)wall_clock64());
@@ -70,7 +75,7 @@ __device__ __forceinline__ void add_work(unsigned long long *work, unsigned long
     if (e) atomicAdd(slot + WORK_EDGES, e);
     if (v) atomicAdd(slot + WORK_VERTS, v);
     // workgroups start in order: the first one of each slot begins it
-    if (blockIdx.x < WORK_SLOTS) atomicMax(slot + WORK_BEGIN, ~t0);
+    if (t0 != NO_STAMP && blockIdx.x < WORK_SLOTS) atomicMax(slot + WORK_BEGIN, ~t0);
     atomicMax(slot + WORK_END, (unsigned long long)wall_clock64());
   }
 }

@@ -349,7 +349,6 @@ __global__ void __launch_bounds__(PB_BLOCK) k_pb_scatter(Bd body, pb_t pb) {
 // in atomics.)
 template <class Bd, typename MSG>
 __global__ void __launch_bounds__(PB_BLOCK) k_pb_gather(Bd body, pb_t pb) {
-  const unsigned long long t0 = wall_clock64();
   using WA = typename Bd::WA;
   constexpr int CAP = PB_LDS_BYTES / (int)sizeof(WA);
   __shared__ WA s_acc[CAP];
@@ -476,8 +475,9 @@ __global__ void __launch_bounds__(PB_BLOCK) k_pb_gather(Bd body, pb_t pb) {
         body.f.compAtomic(body.f.wa_of(lo), tot, body.g);
     }
   }
-  add_work<PB_BLOCK>(body.as.dg_work, t0, threadIdx.x == 0 ? (unsigned long long)(e1 - e0) : 0ull,
-                     0ull);
+  // (the scatter stamped the begin)
+  add_work<PB_BLOCK>(body.as.dg_work, NO_STAMP,
+                     threadIdx.x == 0 ? (unsigned long long)(e1 - e0) : 0ull, 0ull);
 }
 
 // The functor's filter on the targets of split bins (pb_fuse_filter).

@@ -339,6 +339,24 @@ def test_pagerank_eps_after_fixed_iterations(gsw, gset, first, eps):
     g.close()
 
 
+@pytest.mark.parametrize("configs", ["Pull-Bitmap-%s-Standalone" % lb for lb in LBS + ["TWOD"]])
+@pytest.mark.parametrize("pull_kernel", [0, 1, 2])
+def test_expand_times(gsw, gset, monkeypatch, configs, pull_kernel):
+    """Every expand's record has its time, whichever launch stamps its begin
+    and its end, and together they fit the run's device time."""
+    monkeypatch.setenv("GSW_ROWS_EDGES", "0")  # the blocked kernels too
+    _, g = gset["rmat12"]
+    for _ in range(2):
+        g.pagerank(0.85, 6, configs=configs, pull_kernel=pull_kernel)
+        ms = [r["ms"] for r in g.records()]
+        assert len(ms) == 6 and min(ms) > 0
+        assert sum(ms) <= g.last_stats.device_ms
+        for run, k in ((g.delta_pagerank, dict(max_iters=5)), (g.bc, dict(root=3))):
+            run(configs=configs, pull_kernel=pull_kernel, **k)
+            ms = [r["ms"] for r in g.records()]
+            assert ms and min(ms) > 0 and sum(ms) <= g.last_stats.device_ms
+
+
 @pytest.mark.parametrize("slice_kb", [1, 4, 64])
 def test_pagerank_twod_slices(gsw, orc, monkeypatch, slice_kb):
     """TWOD with several source slices (one launch each): R-MAT 12 has
