@@ -21,6 +21,7 @@ using GC = device_graph_t<COO, Empty>;
 
 struct BFS : Functor<VC, int, Empty, Empty> {
   static constexpr bool level_sync = true;
+  static constexpr bool repeatable = true;
   __device__ Status filter(int v, GU g) {
     const int lvl = *wa_of(v);
     if (lvl == g.get_level()) return Active;

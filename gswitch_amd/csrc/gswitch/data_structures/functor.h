@@ -93,6 +93,18 @@ template <typename F>
 struct is_level_sync<F, std::void_t<decltype(F::level_sync)>>
     : std::integral_constant<bool, F::level_sync> {};
 
+// Standalone pushes of a run that prunes by visits (conf_pruning) mark every
+// target, so compAtomic runs once per target. A functor for which running it
+// once per edge is the same (all messages to a target within a level are
+// equal, and its cond refuses a target that an earlier level reached) may
+// declare
+//   static constexpr bool repeatable = true;
+// and its standalone pushes do without the marks.
+template <typename F, typename = void> struct is_repeatable : std::false_type {};
+template <typename F>
+struct is_repeatable<F, std::void_t<decltype(F::repeatable)>>
+    : std::integral_constant<bool, F::repeatable> {};
+
 template <typename WA, typename RA, typename E>
 struct Functor<EC, WA, RA, E> {
   typedef WA wa_t;

@@ -101,12 +101,12 @@ template <typename G, typename F, bool FUSED> struct push_body {
   // true when u must be appended to the next queue (fused only)
   __device__ __forceinline__ bool operator()(int v, int u, int64_t e) {
     if constexpr (!FUSED) {
-      // A level-synchronous functor that prunes by visits is idempotent (BFS):
-      // it writes the same value whichever edge comes first, so its standalone
-      // levels store it without a mark (15 K edges into 4096 vertices: with
-      // the atomics on 64 words the launch took 44 us, without 9).
+      // A repeatable functor (BFS) writes the same value whichever edge comes
+      // first, so its standalone levels store it without a mark (15 K edges
+      // into 4096 vertices: with the atomics on 64 words the launch took
+      // 44 us, without 9).
       bool go = true;
-      if (conf.conf_pruning && !is_level_sync<F>::value)
+      if (conf.conf_pruning && !is_repeatable<F>::value)
         go = as.bitmap.mark_duplicate_lite(u);
       if (go && !conf.conf_toall) go = as.bitmap.is_inactive(u);
       if (go) {

@@ -88,6 +88,27 @@ def test_bfs_application(gsw, orc, mtx, graph, configs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("graph", ["rmat", "grid"])
+@pytest.mark.parametrize("lb", ["TM", "WM", "CM", "STRICT", "TWC"])
+@pytest.mark.parametrize("fmt", ["Queue", "SortedQueue", "Bitmap"])
+def test_pruned_pushes_update_once(gsw, orc, mtx, graph, lb, fmt):
+    """A level-synchronous functor that prunes by visits and declares no more
+    gets compAtomic once per reached vertex from standalone pushes."""
+    h = gsw.read_mtx(mtx[graph], header=True)
+    root = h.max_degree_vertex()
+    out = mtx["dir"] / "visits.bin"
+    run("visits_app", [mtx[graph], "-H", "-r", root, "-c",
+                       "Push-%s-%s-Standalone" % (fmt, lb)], out)
+    got = np.fromfile(out, np.int32)
+    level, hits = got[1::2], got[2::2]
+    ref = orc.bfs(h.row_ptr, h.col, root)
+    assert np.array_equal(level, ref)
+    want = (ref >= 0).astype(np.int32)
+    want[root] = 0
+    assert np.array_equal(hits, want)
+
+
+@pytest.mark.gpu
 def test_bfs_application_random_root(gsw, orc, mtx):
     """No -r: random_root() picks a vertex with edges; the result is that
     root's BFS."""
