@@ -63,7 +63,7 @@ def build_lib(jobs=None):
 
 
 APPS_DIR = os.path.join(REPO, "tests", "apps")
-APPS = ["bfs_app", "sssp_app", "cc_app", "visits_app"]
+APPS = ["bfs_app", "sssp_app", "cc_app", "visits_app", "rank_app"]
 
 
 def build_apps():

@@ -94,6 +94,7 @@ struct PR : Functor<VC, double, float, Empty> {
   // a message is a stored FP32 rank widened to FP64: it is stored exactly
   // as FP32 where messages are staged per edge (propagation blocking)
   using msg_t = float;
+  static constexpr bool ra_pair = true;
   float damp;
   float eps;
   __device__ Status filter(int v, GU g) {

@@ -464,7 +464,7 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
     // a small graph whose every vertex stays active: whole rows, the filter
     // with them (kernels/pull_rows.h), unless the blocked layout is asked for
     bool use_rows = false;
-    if constexpr (pb_has_filter_acc<F>::value)
+    if constexpr (pb_has_filter_acc<F>::value && is_ra_pair<F>::value)
       use_rows = use_pb && conf.counts_known && conf.wa_zero &&
                  g.nedges <= rows_max_edges() && !std::getenv("GSW_PB_ECAP") &&
                  !std::getenv("GSW_PB_GROUPS");
@@ -574,7 +574,7 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
                              dim3(BLOCK), 0, st, body);
           break;
         case TWOD: {
-          if constexpr (pb_has_filter_acc<F>::value) {
+          if constexpr (pb_has_filter_acc<F>::value && is_ra_pair<F>::value) {
             if (use_rows) {
               const rowbins_t &rb = *g.rowbins;
               int4 first;

@@ -105,6 +105,16 @@ template <typename F>
 struct is_repeatable<F, std::void_t<decltype(F::repeatable)>>
     : std::integral_constant<bool, F::repeatable> {};
 
+// An expand may write the read attributes to a second array and exchange the
+// two pointers of the functor object that it was given (the whole-row pull).
+// Copies of the object, such as a driver's own when the loop took it by value,
+// then hold the older array, so this is done only for a functor that declares
+//   static constexpr bool ra_pair = true;
+template <typename F, typename = void> struct is_ra_pair : std::false_type {};
+template <typename F>
+struct is_ra_pair<F, std::void_t<decltype(F::ra_pair)>>
+    : std::integral_constant<bool, F::ra_pair> {};
+
 template <typename WA, typename RA, typename E>
 struct Functor<EC, WA, RA, E> {
   typedef WA wa_t;

@@ -157,3 +157,19 @@ def test_cc_application(gsw, orc, mtx, graph):
     assert "passed" in stdout
     got = np.fromfile(out, np.int32)
     assert np.array_equal(got, orc.cc(h.row_ptr, h.col))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graph", ["rmat", "grid"])
+@pytest.mark.parametrize("iters", [1, 2, 3])
+def test_rank_application(gsw, orc, mtx, graph, iters, monkeypatch):
+    """A functor with filter_acc whose driver takes it by value reads its ranks
+    from the array that it allocated, after odd and even iteration counts."""
+    h = gsw.read_mtx(mtx[graph], header=True)
+    monkeypatch.setenv("GSW_APP_ITERS", str(iters))
+    out = mtx["dir"] / "rank.bin"
+    run("rank_app", [mtx[graph], "-H", "-c", "Pull-Bitmap-TWOD-Standalone"], out)
+    got = np.fromfile(out, np.float32) * np.maximum(h.degrees, 1)
+    ref = orc.pagerank(h.row_ptr, h.col, 0.85, iters)
+    # a rank is rounded to 32 bits per iteration, and its source share once
+    assert np.max(np.abs(got - ref) / ref) <= 2 ** -23 * (iters + 1)
