@@ -36,7 +36,9 @@ struct level_record_t {
   int level;
   int dir, fmt, lb, fused, sorted;
   int kernel;              // pulls: 0 length-binned / merge-path, 1 segmented,
-                           // 2 propagation blocking (pull_kernel in effect)
+                           // 2 propagation blocking or, on a graph it is
+                           // slower for, whole rows (pull_kernel in effect)
+  bool rows;               // whole rows ran: verts is the number of targets
   long long frontier;      // input frontier length (queue) or n (bitmap)
   long long active, inactive;
   long long edges;         // edges inspected by the expand (device counter)
@@ -70,7 +72,7 @@ struct executor_t {
     for (size_t i = 0; i < log.size(); ++i) {
       const unsigned long long *r = w + std::min<size_t>(i, (size_t)rows - 1) * WORK_N;
       log[i].edges = (long long)r[WORK_EDGES];
-      log[i].verts = (long long)r[WORK_VERTS];
+      log[i].verts = log[i].rows ? (long long)as.size : (long long)r[WORK_VERTS];
       // (an expand without a workgroup that counted has no stamps)
       if (profile && r[WORK_END] > ~r[WORK_BEGIN])
         log[i].ms = (float)((double)(r[WORK_END] - ~r[WORK_BEGIN]) / clock_khz);
@@ -227,7 +229,7 @@ struct executor_t {
     }
     if (conf.conf_fuse_inspect && as.queue.mode == Normal)
       as.queue.slot_zero[as.queue.cursor ^ 1] = false;
-    dispatch(as, g, f, conf, stat);
+    rec.rows = dispatch(as, g, f, conf, stat);
     log.push_back(rec);
     if (conf.verbose) {
       std::printf("level %d frontier %lld ", rec.level, rec.frontier);
@@ -399,8 +401,9 @@ struct executor_t {
     return ran;
   }
 
+  // true where the whole-row pull ran
   template <typename G, typename F>
-  void dispatch(active_set_t &as, G &g, F &f, config_t &conf, stat_t &stat);
+  bool dispatch(active_set_t &as, G &g, F &f, config_t &conf, stat_t &stat);
 };
 
 // grid for a frontier of N items processed `per` items per workgroup
@@ -436,7 +439,7 @@ inline int strict_grid(const config_t &conf, int64_t N) {
 }
 
 template <typename G, typename F>
-void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
+bool executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
                           stat_t &stat) {
   using namespace gsw;
   hipStream_t st = stream();
@@ -445,10 +448,10 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
     hipLaunchKernelGGL((k_expand_ec<G, F>), dim3(grid_for(N)), dim3(BLOCK), 0,
                        st, as, g, f);
     H_ERR(hipGetLastError());
-    return;
+    return false;
   } else {
     const int64_t N = as.get_size_host();
-    if (N == 0) return;
+    if (N == 0) return false;
     const bool push = conf.conf_dir == Push;
     const bool fused = conf.conf_fuse_inspect;
     LB lb = conf.conf_lb;
@@ -461,13 +464,15 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
     using MSG = typename pb_msg<F>::type;
     using WAt = typename F::wa_t;
     const bool use_pb = lb == TWOD && conf.pb_pull && g.pb;
-    // a small graph whose every vertex stays active: whole rows, the filter
-    // with them (kernels/pull_rows.h), unless the blocked layout is asked for
+    // every vertex stays active: on graphs that gain by it, whole rows and the
+    // filter with them (kernels/pull_rows.h), unless the blocked layout is
+    // asked for
     bool use_rows = false;
     if constexpr (pb_has_filter_acc<F>::value && is_ra_pair<F>::value)
       use_rows = use_pb && conf.counts_known && conf.wa_zero &&
-                 g.nedges <= rows_max_edges() && !std::getenv("GSW_PB_ECAP") &&
-                 !std::getenv("GSW_PB_GROUPS");
+                 !std::getenv("GSW_PB_ECAP") && !std::getenv("GSW_PB_GROUPS") &&
+                 rows_wanted(*g.rowbins, g.dgr_adj_list, g.nvertexs, g.nedges,
+                             (int)sizeof(typename F::ra_t));
     if (use_rows) {
       rows_ensure(*g.rowbins, g.dgr_row_ptr, g.nvertexs);
       if (!f.data.dg_ra2)
@@ -659,5 +664,6 @@ void executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
       }
       H_ERR(hipGetLastError());
     }
+    return use_rows;
   }
 }

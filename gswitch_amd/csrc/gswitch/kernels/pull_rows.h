@@ -11,10 +11,22 @@
 // level still read the first), which then change places.
 // Latency bounds it: a list entry, row offsets, columns and messages are a
 // chain of four loads.
-// Measured per PageRank iteration, against propagation blocking: R-MAT 11 (26 K
-// edges) 28.8 -> 6.8 us, R-MAT 14 (228 K) 35.6 -> 7.8, a web graph of 728 K
-// edges 20.9 -> 8.4, R-MAT 18 (7.6 M) 57 -> 36; but 16.4 M edges over 2 M
-// sources 82 -> 129 and R-MAT 20 (31 M) 103 -> 179, hence the limit.
+// Which graphs: the gathers gain where they stay in the caches, that is with
+// few sources, with few edges, or with sources that concentrate on part of the
+// lines (hubs with neighbouring ids) or follow the rows (a grid); a sample of
+// the in-edges tells the last (rows_cover). Measured per PageRank iteration, us,
+// propagation blocking -> whole rows:
+//   few sources      uniform random, 64 K of them: 2.1 M edges 22 -> 13, 8.4 M 50 -> 43;
+//                    128 K: 2.1 M 20 -> 17, 4.2 M 25 -> 22, 8.4 M 41 -> 40; but
+//                    256 K: 2.1 M 20 -> 20, 4.2 M 24 -> 29
+//   few edges        random, 1 M sources: 1 M edges 25 -> 17, 2.1 M 26 -> 24, 3.1 M 25 -> 30
+//   concentrated     R-MAT 19 to 22, 7 to 8.3 M edges: 58 -> 38, 71 -> 46, 83 -> 57, 114 -> 76;
+//                    grid 1400 x 1400 78 -> 27
+//   spread           random, 8.4 M edges, 512 K / 1 M / 2 M sources: 39 -> 52, 42 -> 74, 51 -> 104;
+//                    R-MAT 19 to 22 with shuffled ids 36 -> 47, 44 -> 57, 56 -> 72, 81 -> 110;
+//                    preferential attachment, 1 M sources 46 -> 59
+// The sample covers 0.08 (grids) to 0.30 of the lines on the concentrated graphs
+// and 0.45 to 0.63 on the spread ones, hence the line at 3/8.
 #pragma once
 #include "expand_pull.h"
 #include "pb.h"
@@ -24,12 +36,9 @@ namespace gsw {
 constexpr int ROWS_CLASSES = 4;
 constexpr int ROWS_LANE = 8, ROWS_GROUP = 128, ROWS_WAVE = 2048;  // longest row of a class
 constexpr int64_t ROWS_MAX_EDGES = 8 << 20;
-
-// (GSW_ROWS_EDGES: another limit, for sweeps)
-inline int64_t rows_max_edges() {
-  const char *e = std::getenv("GSW_ROWS_EDGES");
-  return e ? std::atoll(e) : ROWS_MAX_EDGES;
-}
+constexpr int64_t ROWS_FEW_SOURCES = 128 << 10, ROWS_FEW_EDGES = 2 << 20;
+constexpr double ROWS_COVER = 0.375;
+constexpr int ROWS_LINE = 128;  // bytes of a cache line
 
 __device__ __forceinline__ int rows_class(int64_t deg) {
   return deg <= ROWS_LANE ? 0 : deg <= ROWS_GROUP ? 1 : deg <= ROWS_WAVE ? 2 : 3;
@@ -90,6 +99,58 @@ inline void rows_ensure(rowbins_t &rb, const int64_t *rows, int64_t n) {
   }
   H_ERR(hipFree(cnt));
   rb.list = list;
+}
+
+// A sample of the in-edges, as many as the source state has lines, one wavefront
+// per window of 64 consecutive ones: *count += lines touched. `bits`: one per
+// line, zero before. Sources spread evenly touch 1 - 1/e = 0.63 of the lines.
+__global__ void __launch_bounds__(BLOCK)
+    k_rows_cover(const int32_t *__restrict__ cols, int64_t m, int64_t windows, int per_line,
+                 uint32_t *bits, unsigned long long *count) {
+  const int64_t w = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> LOG_WAVE;
+  if (w >= windows) return;
+  const int64_t at = windows > 1 ? w * (m - WAVE) / (windows - 1) : 0;
+  const int line = cols[at + lane_id()] / per_line;
+  const uint32_t bit = 1u << (line & 31);
+  const uint64_t first = ballot(!(atomicOr(bits + (line >> 5), bit) & bit));
+  if (lane_id() == 0 && first) atomicAdd(count, (unsigned long long)__popcll(first));
+}
+
+// The share of the source state's lines that the sample touches, once per
+// graph (m >= WAVE; `src_bytes`: of one source's state).
+inline double rows_cover(rowbins_t &rb, const int32_t *cols, int64_t n, int64_t m,
+                         int src_bytes) {
+  if (rb.cover >= 0) return rb.cover;
+  const int per = MAX(1, ROWS_LINE / src_bytes);
+  const int64_t lines = (n + per - 1) / per, words = (lines + 31) / 32 + 1;
+  const int64_t windows = MAX((int64_t)1, MIN(lines, m) / WAVE);
+  unsigned long long *tmp = nullptr, h = 0;  // the count, then the bits
+  H_ERR(hipMalloc((void **)&tmp, sizeof(*tmp) + sizeof(uint32_t) * words));
+  try {
+    uint32_t *bits = (uint32_t *)(tmp + 1);
+    fill_async<uint32_t>((uint32_t *)tmp, 0u, words + 2);
+    hipLaunchKernelGGL(k_rows_cover, dim3((unsigned)((windows * WAVE + BLOCK - 1) / BLOCK)),
+                       dim3(BLOCK), 0, stream(), cols, m, windows, per, bits, tmp);
+    H_ERR(hipGetLastError());
+    H_ERR(hipMemcpyAsync(&h, tmp, sizeof(h), hipMemcpyDeviceToHost, stream()));
+    sync();
+  } catch (...) {
+    (void)hipFree(tmp);
+    throw;
+  }
+  H_ERR(hipFree(tmp));
+  return rb.cover = (double)h / (double)lines;
+}
+
+// Whether whole rows are the faster pull of a graph (the reasons and both
+// sides' times are above). GSW_ROWS_EDGES: by that number of edges alone, for
+// sweeps.
+inline bool rows_wanted(rowbins_t &rb, const int32_t *cols, int64_t n, int64_t m,
+                        int src_bytes) {
+  if (const char *e = std::getenv("GSW_ROWS_EDGES")) return m <= std::atoll(e);
+  if (m > ROWS_MAX_EDGES) return false;
+  if (n <= ROWS_FEW_SOURCES || m <= ROWS_FEW_EDGES) return true;
+  return rows_cover(rb, cols, n, m, src_bytes) < ROWS_COVER;
 }
 
 // workgroups of each class

@@ -124,7 +124,9 @@ typedef struct {
                           length-binned source slices, STRICT as a merge-path
                           walk; 1 both as segmented reductions; 2 (default)
                           TWOD by propagation blocking (LDS-sized source
-                          chunks and target bins), STRICT as in 0 */
+                          chunks and target bins) or, for PageRank with
+                          eps = 0 on graphs that gain by it, by whole rows
+                          (records then give verts = n); STRICT as in 0 */
   int32_t capture;     /* gsw_bfs_multi: >0 = hipGraph-captured fused level loop,
                           2*capture levels per replay; 0 = per-level host loop */
   int32_t grid;        /* gsw_bfs_multi captured loop: workgroups per launch
@@ -157,7 +159,7 @@ typedef struct {
   int64_t active;   /* active vertices (edges for CC) at this level */
   int64_t inactive;
   int64_t edges;    /* edges inspected by the expand */
-  int64_t verts;    /* frontier vertices expanded */
+  int64_t verts;    /* frontier vertices expanded (0 where not counted) */
   float ms;         /* expand duration (0 unless profile) */
   float pad2;
 } gsw_level_record;

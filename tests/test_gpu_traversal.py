@@ -312,6 +312,29 @@ def test_pagerank_whole_rows(gsw, orc, monkeypatch, directed):
     g.close()
 
 
+@pytest.mark.parametrize("spec,whole", [("grid", True), ("random", False), ("fewer edges", True),
+                                        ("fewer sources", True), ("rmat", True)])
+def test_pagerank_pull_follows_locality(gsw, orc, spec, whole):
+    """More than 128 K vertices and 2 Mi edges: whole rows where the sources
+    stay in the caches (a grid; R-MAT's hubs), the blocked layout where every
+    in-edge reads another line, and whole rows again on one side of either
+    bound."""
+    rng = np.random.default_rng(2)
+    def random(n, m):
+        return gsw.from_edges(n, rng.integers(0, n, m), rng.integers(0, n, m))
+    n, m = (128 << 10) + 1, (2 << 20) // 2 + 400
+    h = {"grid": lambda: gsw.grid2d(800, 810, 0.1, 0.01, 3), "random": lambda: random(n, m),
+         "fewer edges": lambda: random(n, m - 400), "fewer sources": lambda: random(n - 1, m),
+         "rmat": lambda: gsw.rmat(19, 3, seed=2)}[spec]()
+    assert (h.m <= 2 << 20) == (spec == "fewer edges")
+    g = gsw.Graph(h)
+    for iters in (3, 4):
+        pr = g.pagerank(0.85, iters, configs="Pull-Bitmap-TWOD-Standalone")
+        assert max_rel(pr, orc.pagerank(h.row_ptr, h.col, 0.85, iters)) <= PR_TOL
+        assert [r["verts"] for r in g.records()] == [h.n if whole else 0] * iters
+    g.close()
+
+
 @pytest.mark.parametrize("first", [dict(configs="Pull-Queue-WM-Standalone"),
                                    dict(configs="Push-Bitmap-STRICT-Standalone"),
                                    dict(pull_kernel=0), dict(pull_kernel=1)])
