@@ -38,8 +38,10 @@ constexpr int CC_HALVE_AFTER = 16;  // steps of a link before it halves its path
 constexpr int CC_HOPS = 4;          // first neighbours a vertex follows at the start
 constexpr int CC_SILP = 4;          // vertices a lane samples at once
 
-// A parent pointer, possibly an old one from this XCD's L2: pointers only move
-// to smaller ancestors within a launch, so an old value is an ancestor too.
+// A parent pointer, possibly an old one from this XCD's L2: every value that an
+// entry ever holds is an ancestor of its vertex, so an old one is too (a store
+// that halves a path may even put a larger ancestor back), and a hooked vertex
+// that still looks like a root fails its CAS.
 // (Loads that are coherent over the device cost more: 2 M-vertex random graph
 // of mean degree 6, whole CC 276 against 303 us.)
 __device__ __forceinline__ int cc_get(const int *p, int64_t i) {
@@ -56,20 +58,28 @@ __device__ __forceinline__ int cc_get(const int *p, int64_t i) {
 // 0.47 ms with it), while on random graphs and R-MAT walks are short and the
 // stores of halving at once cost more than they save (the random graph above:
 // after 2 steps 1110 us, after 8 370, after 16 or never 277).
-__device__ __forceinline__ void cc_link(int a, int b, int *p) {
+// `fresh`: whether the larger side is a root is looked up past the caches.
+// Directed graphs need it: their starts leave trees whose roots many lanes hook
+// at once, and every lane that saw an old root would queue an atomic on it
+// (R-MAT 20 with half its edges, directed: the second neighbours' links took
+// 406 us). Undirected random graphs are 10 % slower with it. Returns an ancestor of both, near the root, for the
+// next link of a row.
+__device__ __forceinline__ int cc_link(int a, int b, int *p, bool fresh) {
   for (int step = 0; a != b; ++step) {
     const int hi = a > b ? a : b, lo = a > b ? b : a;
-    int ph = cc_get(p, hi);
-    if (ph == lo) return;
+    int ph = fresh ? __hip_atomic_load(p + hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                   : cc_get(p, hi);
+    if (ph == lo) return lo;
     if (ph == hi) {
       ph = atomicCAS(p + hi, hi, lo);
-      if (ph == hi) return;
+      if (ph == hi) return lo;
     }
     a = cc_get(p, ph);
     if (step >= CC_HALVE_AFTER)
       __hip_atomic_store(p + hi, a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     b = cc_get(p, lo);
   }
+  return a;
 }
 
 // Where v hooks at the start: the smallest vertex within CC_HOPS steps over
@@ -96,11 +106,15 @@ __global__ void __launch_bounds__(BLOCK)
     p[v] = cc_start_of((int)v, first);
 }
 
-// link every vertex with its second neighbour (with `skip_lv`, only the
-// vertices whose skip_lv entry is negative)
+// Link every vertex with its second neighbour, or with its only one where that
+// is larger, so that k_cc_start did not hook it (with `skip_lv`, only the
+// vertices whose skip_lv entry is negative). Without the latter a star whose
+// hub has the largest id was left to k_cc_rest, where one wavefront walked the
+// hub: 1 M leaves 11.1 ms, now 0.04.
 __global__ void __launch_bounds__(BLOCK)
     k_cc_sample(const int64_t *__restrict__ rows, const int32_t *__restrict__ cols,
-                int64_t n, int *p, const int *__restrict__ skip_lv) {
+                int64_t n, int *p, const int *__restrict__ skip_lv,
+                bool fresh) {
   const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t v0 = tid; v0 < n; v0 += stride * CC_SILP) {
@@ -109,27 +123,31 @@ __global__ void __launch_bounds__(BLOCK)
     // whole CC 277 -> 257 and 223 -> 180 us against one vertex at a time)
     int a[CC_SILP], b[CC_SILP];
     int64_t s[CC_SILP];
+    bool only[CC_SILP];
 #pragma unroll
     for (int k = 0; k < CC_SILP; ++k) {
       const int64_t v = v0 + k * stride;
       s[k] = -1;
+      only[k] = false;
       if (v < n && !(skip_lv && skip_lv[v] >= 0)) {
-        const int64_t r = rows[v];
-        if (rows[v + 1] - r > 1) s[k] = r + 1;
+        const int64_t r = rows[v], e = rows[v + 1];
+        only[k] = e - r == 1;
+        if (e > r) s[k] = only[k] ? r : r + 1;
       }
     }
 #pragma unroll
     for (int k = 0; k < CC_SILP; ++k) a[k] = s[k] >= 0 ? cols[s[k]] : 0;
 #pragma unroll
     for (int k = 0; k < CC_SILP; ++k) {
-      b[k] = 0;
-      if (s[k] >= 0) {
+      const int64_t v = v0 + k * stride;
+      b[k] = a[k];
+      if (s[k] >= 0 && !(only[k] && a[k] < v)) {
         a[k] = cc_get(p, a[k]);
-        b[k] = cc_get(p, v0 + k * stride);
+        b[k] = cc_get(p, v);
       }
     }
 #pragma unroll
-    for (int k = 0; k < CC_SILP; ++k) cc_link(a[k], b[k], p);
+    for (int k = 0; k < CC_SILP; ++k) (void)cc_link(a[k], b[k], p, fresh);
   }
 }
 
@@ -304,7 +322,7 @@ __global__ void __launch_bounds__(BLOCK)
     k_cc_rest(const int64_t *__restrict__ rows, const int32_t *__restrict__ cols,
               int64_t n, int skip_arg, const int *skip_dev,
               const int64_t *__restrict__ off, int64_t count, int *p,
-              int disjoint) {
+              int disjoint, bool fresh) {
   const int skip_root = skip_dev ? *skip_dev : skip_arg;
   const int lane = lane_id();
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> LOG_WAVE;
@@ -313,10 +331,11 @@ __global__ void __launch_bounds__(BLOCK)
     const int64_t v = base + lane;
     int64_t s = 0, e = 0, lo = 0, hi = 0;
     bool in_s = false;
+    int root = 0;
     if (v < n) {
       s = rows[v];
       e = rows[v + 1];
-      const int root = cc_get(p, v);
+      root = cc_get(p, v);
       if (skip_root >= 0) {
         in_s = root == skip_root;
         hi = n;
@@ -334,7 +353,7 @@ __global__ void __launch_bounds__(BLOCK)
     if (!wide)
       for (int64_t j = s; j < e; ++j) {
         const int u = cols[j];
-        if (!in_s || u < lo || u >= hi) cc_link((int)v, u, p);
+        if (!in_s || u < lo || u >= hi) root = cc_link(root, cc_get(p, u), p, fresh);
       }
     uint64_t wmask = ballot(wide);
     while (wmask) {
@@ -343,10 +362,10 @@ __global__ void __launch_bounds__(BLOCK)
       const int64_t ws = __shfl(s, w, 64), we = __shfl(e, w, 64);
       const int64_t wl = __shfl(lo, w, 64), wh = __shfl(hi, w, 64);
       const bool wi = __shfl((int)in_s, w, 64) != 0;
-      const int wv = (int)(base + w);
+      int wr = __shfl(root, w, 64);
       for (int64_t j = ws + lane; j < we; j += WAVE) {
         const int u = cols[j];
-        if (!wi || u < wl || u >= wh) cc_link(wv, u, p);
+        if (!wi || u < wl || u >= wh) wr = cc_link(wr, cc_get(p, u), p, fresh);
       }
     }
   }

@@ -10,6 +10,8 @@ import itertools
 
 import numpy as np
 import pytest
+from scipy.sparse import coo_matrix
+from scipy.sparse.csgraph import connected_components
 
 from conftest import csr_from_edges
 
@@ -256,6 +258,52 @@ def test_cc_long_chains_and_samples(gsw, orc, shape):
     h = gsw.from_edges(n, e[:, 0], e[:, 1])
     g = gsw.Graph(h)
     assert np.array_equal(g.cc(), orc.cc(h.row_ptr, h.col))
+    g.close()
+
+
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("shape", ["star_last", "star_middle", "pairs", "two_hubs", "chain_of_stars",
+                                   "rmat_reversed", "rmat_half"])
+def test_cc_hubs_anywhere(gsw, shape, directed):
+    """Vertices whose only neighbour is larger (a hub with the largest id or
+    one in the middle, pairs), hubs that only second neighbours lead to, and
+    R-MAT with its hubs at the other end or with each edge in one direction."""
+    rng = np.random.default_rng(11)
+    n = 5000
+    if shape in ("star_last", "star_middle"):
+        hub = n - 1 if shape == "star_last" else n // 2
+        leaf = np.delete(np.arange(n), hub)
+        e = np.stack([leaf, np.full(n - 1, hub)], 1)
+    elif shape == "pairs":
+        ids = rng.permutation(n)
+        e = ids.reshape(-1, 2)
+    elif shape == "two_hubs":
+        leaf = np.arange(n - 2)
+        e = np.concatenate([np.stack([leaf, np.full(n - 2, h)], 1) for h in (n - 2, n - 1)])
+    elif shape == "chain_of_stars":  # hubs last, their leaves' ids interleaved
+        hub = n - 50 + np.arange(n - 50) % 50
+        e = np.concatenate([np.stack([np.arange(n - 50), hub], 1),
+                            np.stack([np.arange(n - 50, n - 1), np.arange(n - 49, n)], 1)])
+    else:
+        h = gsw.rmat(13, 6, seed=7)
+        n = h.n
+        src = np.repeat(np.arange(n), np.diff(h.row_ptr))
+        keep = src < h.col
+        e = np.stack([src[keep], h.col[keep]], 1)
+        flip = rng.random(len(e)) < 0.5
+        e[flip] = e[flip][:, ::-1]
+        if shape == "rmat_reversed":
+            e = n - 1 - e
+    if directed and shape != "rmat_half":
+        e = e[:, ::-1] if shape in ("star_middle", "two_hubs") else e
+    h = gsw.from_edges(n, e[:, 0], e[:, 1], directed=directed)
+    _, comp = connected_components(coo_matrix((np.ones(len(e)), (e[:, 0], e[:, 1])), (n, n)),
+                                   directed=True, connection="weak")
+    first = np.full(comp.max() + 1, n)
+    np.minimum.at(first, comp, np.arange(n))
+    g = gsw.Graph(h)
+    for _ in range(2):
+        assert np.array_equal(g.cc(), first[comp])
     g.close()
 
 
