@@ -471,7 +471,7 @@ bool executor_t::dispatch(active_set_t &as, G &g, F &f, config_t &conf,
     if constexpr (pb_has_filter_acc<F>::value && is_ra_pair<F>::value)
       use_rows = use_pb && conf.counts_known && conf.wa_zero &&
                  !std::getenv("GSW_PB_ECAP") && !std::getenv("GSW_PB_GROUPS") &&
-                 rows_wanted(*g.rowbins, g.dgr_adj_list, g.nvertexs, g.nedges,
+                 rows_wanted(*g.rowbins, g.dgr_row_ptr, g.dgr_adj_list, g.nvertexs, g.nedges,
                              (int)sizeof(typename F::ra_t));
     if (use_rows) {
       rows_ensure(*g.rowbins, g.dgr_row_ptr, g.nvertexs);

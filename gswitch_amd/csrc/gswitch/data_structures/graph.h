@@ -154,7 +154,8 @@ struct pb_t {
 struct rowbins_t {
   int32_t *list = nullptr;  // [n], class k from off[k] on
   int64_t off[4] = {0, 0, 0, 0}, cnt[4] = {0, 0, 0, 0};
-  double cover = -1;  // rows_cover(), once known
+  int64_t longest = -1;  // longest row (0: none above ROWS_WAVE), once counted
+  double cover = -1;     // rows_cover(), once known
 };
 
 template <GraphFmt fmt, typename E> struct device_graph_t {};

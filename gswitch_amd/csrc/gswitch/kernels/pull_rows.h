@@ -27,6 +27,10 @@
 //                    preferential attachment, 1 M sources 46 -> 59
 // The sample covers 0.08 (grids) to 0.30 of the lines on the concentrated graphs
 // and 0.45 to 0.63 on the spread ones, hence the line at 3/8.
+// Not where one row is long, since one workgroup walks it, 0.6 us per 1024
+// edges, while propagation blocking splits it. Stars: 16 K leaves 35 -> 14, 32 K
+// 34 -> 23, 65 K 35 -> 43, 262 K 36 -> 161; a row of 1/128 of all edges ends with
+// the others.
 #pragma once
 #include "expand_pull.h"
 #include "pb.h"
@@ -37,6 +41,7 @@ constexpr int ROWS_CLASSES = 4;
 constexpr int ROWS_LANE = 8, ROWS_GROUP = 128, ROWS_WAVE = 2048;  // longest row of a class
 constexpr int64_t ROWS_MAX_EDGES = 8 << 20;
 constexpr int64_t ROWS_FEW_SOURCES = 128 << 10, ROWS_FEW_EDGES = 2 << 20;
+constexpr int64_t ROWS_LONGEST = 32 << 10;
 constexpr double ROWS_COVER = 0.375;
 constexpr int ROWS_LINE = 128;  // bytes of a cache line
 
@@ -44,8 +49,9 @@ __device__ __forceinline__ int rows_class(int64_t deg) {
   return deg <= ROWS_LANE ? 0 : deg <= ROWS_GROUP ? 1 : deg <= ROWS_WAVE ? 2 : 3;
 }
 
-// pass 0: class sizes into cnt[0..4); pass 1: rows into list, class k from
-// cnt[k] on (the offsets, moved along)
+// pass 0: class sizes into cnt[0..4), the longest row above ROWS_WAVE into
+// cnt[4]; pass 1: rows into list, class k from cnt[k] on (the offsets, moved
+// along)
 __global__ void __launch_bounds__(BLOCK)
     k_rows_list(const int64_t *__restrict__ rows, int64_t n, int32_t *list,
                 unsigned long long *cnt) {
@@ -54,7 +60,9 @@ __global__ void __launch_bounds__(BLOCK)
   const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> LOG_WAVE;
   for (int64_t base = wave << 6; base < n; base += nwaves << 6) {
     const int64_t v = base + lane;
-    const int c = v < n ? rows_class(rows[v + 1] - rows[v]) : -1;
+    const int64_t deg = v < n ? rows[v + 1] - rows[v] : -1;
+    const int c = v < n ? rows_class(deg) : -1;
+    if (!list && deg > ROWS_WAVE) atomicMax(cnt + ROWS_CLASSES, (unsigned long long)deg);
 #pragma unroll
     for (int k = 0; k < ROWS_CLASSES; ++k) {
       const uint64_t m = ballot(c == k);
@@ -67,29 +75,45 @@ __global__ void __launch_bounds__(BLOCK)
   }
 }
 
-inline void rows_ensure(rowbins_t &rb, const int64_t *rows, int64_t n) {
-  if (rb.list) return;
-  unsigned long long *cnt = nullptr, h[ROWS_CLASSES];
-  int32_t *list = nullptr;
+// class sizes and the longest row, once per graph
+inline void rows_count(rowbins_t &rb, const int64_t *rows, int64_t n) {
+  if (rb.longest >= 0) return;
+  unsigned long long *cnt = nullptr, h[ROWS_CLASSES + 1];
   H_ERR(hipMalloc((void **)&cnt, sizeof(h)));
   try {
-    H_ERR(hipMalloc((void **)&list, sizeof(int32_t) * (n + 1)));
-    const dim3 grid(grid_for((n + 63) / 64 * 64));
-    fill_async<unsigned long long>(cnt, 0ull, ROWS_CLASSES);
-    hipLaunchKernelGGL(k_rows_list, grid, dim3(BLOCK), 0, stream(), rows, n,
-                       (int32_t *)nullptr, cnt);
+    fill_async<unsigned long long>(cnt, 0ull, ROWS_CLASSES + 1);
+    hipLaunchKernelGGL(k_rows_list, dim3(grid_for((n + 63) / 64 * 64)), dim3(BLOCK), 0, stream(),
+                       rows, n, (int32_t *)nullptr, cnt);
+    H_ERR(hipGetLastError());
     H_ERR(hipMemcpyAsync(h, cnt, sizeof(h), hipMemcpyDeviceToHost, stream()));
     sync();
-    unsigned long long off[ROWS_CLASSES], at = 0;
-    for (int k = 0; k < ROWS_CLASSES; ++k) {
-      off[k] = at;
-      rb.off[k] = (int64_t)at;
-      rb.cnt[k] = (int64_t)h[k];
-      at += h[k];
-    }
-    GSW_REQUIRE((int64_t)at == n, E_INTERNAL_CHECK, "row classes miss rows");
+  } catch (...) {
+    (void)hipFree(cnt);
+    throw;
+  }
+  H_ERR(hipFree(cnt));
+  int64_t at = 0;
+  for (int k = 0; k < ROWS_CLASSES; ++k) {
+    rb.off[k] = at;
+    rb.cnt[k] = (int64_t)h[k];
+    at += rb.cnt[k];
+  }
+  GSW_REQUIRE(at == n, E_INTERNAL_CHECK, "row classes miss rows");
+  rb.longest = (int64_t)h[ROWS_CLASSES];
+}
+
+inline void rows_ensure(rowbins_t &rb, const int64_t *rows, int64_t n) {
+  if (rb.list) return;
+  rows_count(rb, rows, n);
+  unsigned long long *cnt = nullptr, off[ROWS_CLASSES];
+  for (int k = 0; k < ROWS_CLASSES; ++k) off[k] = (unsigned long long)rb.off[k];
+  int32_t *list = nullptr;
+  H_ERR(hipMalloc((void **)&cnt, sizeof(off)));
+  try {
+    H_ERR(hipMalloc((void **)&list, sizeof(int32_t) * (n + 1)));
     H_ERR(hipMemcpyAsync(cnt, off, sizeof(off), hipMemcpyHostToDevice, stream()));
-    hipLaunchKernelGGL(k_rows_list, grid, dim3(BLOCK), 0, stream(), rows, n, list, cnt);
+    hipLaunchKernelGGL(k_rows_list, dim3(grid_for((n + 63) / 64 * 64)), dim3(BLOCK), 0, stream(),
+                       rows, n, list, cnt);
     H_ERR(hipGetLastError());
     sync();
   } catch (...) {
@@ -145,10 +169,12 @@ inline double rows_cover(rowbins_t &rb, const int32_t *cols, int64_t n, int64_t 
 // Whether whole rows are the faster pull of a graph (the reasons and both
 // sides' times are above). GSW_ROWS_EDGES: by that number of edges alone, for
 // sweeps.
-inline bool rows_wanted(rowbins_t &rb, const int32_t *cols, int64_t n, int64_t m,
-                        int src_bytes) {
+inline bool rows_wanted(rowbins_t &rb, const int64_t *rows, const int32_t *cols, int64_t n,
+                        int64_t m, int src_bytes) {
   if (const char *e = std::getenv("GSW_ROWS_EDGES")) return m <= std::atoll(e);
   if (m > ROWS_MAX_EDGES) return false;
+  rows_count(rb, rows, n);
+  if (rb.longest > MAX(ROWS_LONGEST, m / 128)) return false;
   if (n <= ROWS_FEW_SOURCES || m <= ROWS_FEW_EDGES) return true;
   return rows_cover(rb, cols, n, m, src_bytes) < ROWS_COVER;
 }

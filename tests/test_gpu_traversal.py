@@ -361,20 +361,24 @@ def test_pagerank_whole_rows(gsw, orc, monkeypatch, directed):
 
 
 @pytest.mark.parametrize("spec,whole", [("grid", True), ("random", False), ("fewer edges", True),
-                                        ("fewer sources", True), ("rmat", True)])
+                                        ("fewer sources", True), ("rmat", True),
+                                        ("hub", True), ("larger hub", False)])
 def test_pagerank_pull_follows_locality(gsw, orc, spec, whole):
     """More than 128 K vertices and 2 Mi edges: whole rows where the sources
     stay in the caches (a grid; R-MAT's hubs), the blocked layout where every
     in-edge reads another line, and whole rows again on one side of either
-    bound."""
+    bound, unless one row is too long for a workgroup."""
     rng = np.random.default_rng(2)
     def random(n, m):
         return gsw.from_edges(n, rng.integers(0, n, m), rng.integers(0, n, m))
+    def star(leaves):
+        return gsw.from_edges(leaves + 2, np.full(leaves, leaves + 1), np.arange(leaves))
     n, m = (128 << 10) + 1, (2 << 20) // 2 + 400
     h = {"grid": lambda: gsw.grid2d(800, 810, 0.1, 0.01, 3), "random": lambda: random(n, m),
          "fewer edges": lambda: random(n, m - 400), "fewer sources": lambda: random(n - 1, m),
+         "hub": lambda: star(32 << 10), "larger hub": lambda: star((32 << 10) + 1),
          "rmat": lambda: gsw.rmat(19, 3, seed=2)}[spec]()
-    assert (h.m <= 2 << 20) == (spec == "fewer edges")
+    assert (h.m <= 2 << 20) == (spec in ("fewer edges", "hub", "larger hub"))
     g = gsw.Graph(h)
     for iters in (3, 4):
         pr = g.pagerank(0.85, iters, configs="Pull-Bitmap-TWOD-Standalone")
