@@ -309,11 +309,13 @@ struct executor_t {
     const ahead_t *ha = (const ahead_t *)h;
     uint64_t *const bits[2] = {as.bitmap.visited.dg_bits, as.ahead_bits.dg_bits};
     const int64_t n_bits = prune ? 0 : as.bitmap.visited.n_words;
-    // the exit rule of expand(), on device times: the host's share of a level
-    // (about 25 us there) counts in its average, hence the allowance
+    // the exit rule of expand(): a level's device time, with the host's share
+    // that its levels have (about 25 us), against the average of the levels
+    // before it, expand()'s included
     const bool rule = fets.pattern == Idem && !conf.force.has_fusion;
-    const double allow = clock_khz * 0.1;
-    double ticks = 0;
+    const double share = clock_khz * 0.025;
+    double levels = (double)MAX(1, g.level);
+    double ticks = fets.avg_expand_time * clock_khz * levels;
     const int per = BLOCK / (WAVE / conf.wm_vpw);  // frontier vertices per workgroup
     const double size = (double)as.size;
     int ran = 0, in_buf = q.cursor ^ 1;  // buffer of the next input
@@ -324,17 +326,23 @@ struct executor_t {
       int k = (int)MIN((int64_t)AHEAD, max_levels - ran);
       k = (int)MIN((int64_t)k, (int64_t)WORK_ROWS - 1 - (int64_t)log.size());
       if (k <= 0) break;
-      // grids for twice the growth seen last; an explosion (a random graph's)
-      // is followed level by level once it reaches a good part of the graph
+      // Grids for twice the growth seen last (four times where it is fast). A
+      // level that outgrows its grid is launched again: a second round of a
+      // grid's wavefronts costs more (a tree of fan-out 16 from three roots,
+      // 4124 vertices: 84 us, 193 on a grid of a third). An explosion (a
+      // random graph's) is followed level by level once it reaches a good
+      // part of the graph, and from the start where it is so steep that its
+      // second level may be one for the exit rule (a tree of fan-out 64: 308
+      // us with the rule, 540 when its three levels ran as one batch).
+      const double margin = growth > 2 ? 4 : 2;
       int grids[AHEAD];
       double est = (double)nq, reach[AHEAD];
       for (int j = 0; j < k; ++j) {
-        const double up = j == 0 ? est : MIN(size, 2 * est);
+        const double up = j == 0 ? est : MIN(size, margin * est);
         grids[j] = (int)MAX(1.0, MIN((double)MAX_GRID, std::ceil(up / per)));
-        reach[j] = grids[j] >= MAX_GRID ? 2147483647.0
-                                        : MIN(2147483647.0, MAX(up, 4.0 * grids[j] * per));
+        reach[j] = grids[j] >= MAX_GRID ? 2147483647.0 : (double)grids[j] * per;
         est = MIN(size, est * MAX(growth, 1.25));
-        if (growth > 2 && est * 32 > size) k = j + 1;
+        if ((growth > 2 && est * 32 > size) || growth > 20) k = j + 1;
       }
       if (begin)
         hipLaunchKernelGGL(k_ahead_begin, dim3(grid_for(ran == 0 ? n_bits : 1)), dim3(BLOCK),
@@ -376,9 +384,10 @@ struct executor_t {
         log.push_back(rec);
         ++done;
         const double dt =
-            (double)((j + 1 < k ? ha->clock[j + 1] : h[AHEAD_WORDS]) - ha->clock[j]);
-        if (rule && ran + done > 1 && dt > 5 * (ticks / (ran + done - 1)) + allow) slow = true;
+            share + (double)((j + 1 < k ? ha->clock[j + 1] : h[AHEAD_WORDS]) - ha->clock[j]);
+        if (rule && dt > 5 * (ticks / levels)) slow = true;
         ticks += dt;
+        levels += 1;
       }
       nq = done < k ? ha->sizes[done] : ha->q[(ran + k) % AHEAD_SLOTS];
       if (done > 0) growth = (double)nq / (double)log.back().frontier;

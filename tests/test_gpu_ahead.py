@@ -61,6 +61,28 @@ def test_bfs_queue_outgrows_its_grid(gsw, orc, fan, depth, configs):
     g.close()
 
 
+@pytest.mark.parametrize("fan,depth", [(20, 3), (24, 3), (64, 2), (64, 3)])
+def test_steep_growth_level_by_level(gsw, orc, fan, depth):
+    """Growth above the limit of a batch: one level per batch, with or without
+    leaving the fused mode after it."""
+    h = tree(gsw, fan, depth)
+    src = np.repeat(np.arange(h.n), np.diff(h.row_ptr))
+    up = src < h.col
+    w = np.random.default_rng(fan).integers(1, 65, int(up.sum())).astype(np.uint32)
+    hw = gsw.from_edges(h.n, src[up], h.col[up], w)
+    g = gsw.Graph(hw)
+    for root in (0, 1, h.n - 1):
+        for _ in range(2):
+            assert np.array_equal(g.bfs(root), orc.bfs(h.row_ptr, h.col, root))
+            assert np.array_equal(g.sssp(root), orc.spfa(hw.row_ptr, hw.col, hw.w, root))
+    roots = [0, h.n // 2, h.n - 1]
+    far = np.iinfo(np.int32).max
+    each = [orc.bfs(h.row_ptr, h.col, r) for r in roots]
+    want = np.min([np.where(x < 0, far, x) for x in each], axis=0)
+    assert np.array_equal(g.bfs_multi(roots), want)
+    g.close()
+
+
 @pytest.mark.parametrize("limit", [1, 2, 5, 9, 10, 30])
 def test_bfs_level_limit(gsw, orc, limit):
     h = path(gsw, 60)
