@@ -1040,8 +1040,7 @@ void cc_sample_phase(const gsw_graph *G, int32_t *lab, const int32_t *skip_lv,
   hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(BLOCK), 0, st, lab, n);
   hipLaunchKernelGGL(k_cc_sample, dim3(grid), dim3(BLOCK), 0, st,
                      (const int64_t *)G->dg.dg_row_ptr,
-                     (const int32_t *)G->dg.dg_adj_list, n, lab, (const int *)skip_lv,
-                     G->hg.directed);
+                     (const int32_t *)G->dg.dg_adj_list, n, lab, (const int *)skip_lv);
   hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(BLOCK), 0, st, lab, n);
   H_ERR(hipGetLastError());
 }
@@ -1055,7 +1054,7 @@ void cc_finish_phase(const gsw_graph *G, int32_t *lab, int skip_root,
   hipLaunchKernelGGL(k_cc_rest, dim3(grid_for((n + 63) / 64 * 64)), dim3(BLOCK), 0,
                      st, (const int64_t *)G->dg.dg_row_ptr,
                      (const int32_t *)G->dg.dg_adj_list, n, skip_root, skip_dev,
-                     off, count, lab, 0, G->hg.directed);
+                     off, count, lab, 0);
   hipLaunchKernelGGL(k_cc_compress, dim3(grid_for(n)), dim3(BLOCK), 0, st, lab, n);
   H_ERR(hipGetLastError());
 }
@@ -1125,7 +1124,7 @@ void cc_batched_from_levels(gsw_graph *G, int64_t count, const int32_t *lv) {
   hipLaunchKernelGGL(k_cc_rest, dim3(grid_for((n + 63) / 64 * 64)), dim3(BLOCK), 0, st,
                      (const int64_t *)G->dg.dg_row_ptr, (const int32_t *)G->dg.dg_adj_list,
                      n, -1, (const int *)nullptr, (const int64_t *)G->inst_off, count,
-                     lab, 1, G->hg.directed);
+                     lab, 1);
   hipLaunchKernelGGL(k_cc_compress, dim3(grid_for(n)), dim3(BLOCK), 0, st, lab, n);
   H_ERR(hipGetLastError());
 }

@@ -14,7 +14,8 @@
 // can live in a captured graph):
 //  1. start: every vertex hooks under a smaller vertex it reaches over first
 //     (smallest) in-neighbours, with a plain store (k_cc_start), compress;
-//  2. sampling: every vertex links its second neighbour, compress;
+//  2. sampling: every vertex links its second neighbour (or its only one,
+//     where that is larger), compress;
 //  3. skip set S: vertices whose root is a chosen root -- the most frequent
 //     root of a vertex sample for one graph, or each instance's first vertex
 //     (its smallest id) for a disjoint batch. Vertices outside S link all
@@ -58,21 +59,32 @@ __device__ __forceinline__ int cc_get(const int *p, int64_t i) {
 // 0.47 ms with it), while on random graphs and R-MAT walks are short and the
 // stores of halving at once cost more than they save (the random graph above:
 // after 2 steps 1110 us, after 8 370, after 16 or never 277).
-// `fresh`: whether the larger side is a root is looked up past the caches.
-// Directed graphs need it: their starts leave trees whose roots many lanes hook
-// at once, and every lane that saw an old root would queue an atomic on it
-// (R-MAT 20 with half its edges, directed: the second neighbours' links took
-// 406 us). Undirected random graphs are 10 % slower with it. Returns an ancestor of both, near the root, for the
-// next link of a row.
-__device__ __forceinline__ int cc_link(int a, int b, int *p, bool fresh) {
+// Lanes of a wavefront at one apparent root send one CAS: with one each, every
+// lane that still sees a hooked root as a root queues an atomic on it (two hubs
+// over the same 262 K leaves: 2000 us, so 111; R-MAT 20 with half its edges,
+// directed: the second neighbours' links 406 us). Returns an ancestor of both,
+// near the root, for the next link of a row.
+__device__ __forceinline__ int cc_link(int a, int b, int *p) {
   for (int step = 0; a != b; ++step) {
     const int hi = a > b ? a : b, lo = a > b ? b : a;
-    int ph = fresh ? __hip_atomic_load(p + hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                   : cc_get(p, hi);
+    int ph = cc_get(p, hi);
     if (ph == lo) return lo;
     if (ph == hi) {
-      ph = atomicCAS(p + hi, hi, lo);
-      if (ph == hi) return lo;
+      // the lanes at the first lane's root go on from where its leader found
+      // or hooked that root
+      const int h0 = __builtin_amdgcn_readfirstlane(hi);
+      const int leader = __builtin_ctzll(ballot(hi == h0));
+      const bool mine = hi != h0 || lane_id() == leader;
+      int old = hi;
+      if (mine) old = atomicCAS(p + hi, hi, lo);
+      const int o0 = readlane(old, leader), l0 = readlane(lo, leader);
+      if (mine) {
+        ph = old;
+        if (ph == hi) return lo;
+      } else {
+        ph = o0 == hi ? l0 : o0;
+        if (ph == lo) return lo;
+      }
     }
     a = cc_get(p, ph);
     if (step >= CC_HALVE_AFTER)
@@ -113,8 +125,7 @@ __global__ void __launch_bounds__(BLOCK)
 // hub: 1 M leaves 11.1 ms, now 0.04.
 __global__ void __launch_bounds__(BLOCK)
     k_cc_sample(const int64_t *__restrict__ rows, const int32_t *__restrict__ cols,
-                int64_t n, int *p, const int *__restrict__ skip_lv,
-                bool fresh) {
+                int64_t n, int *p, const int *__restrict__ skip_lv) {
   const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t v0 = tid; v0 < n; v0 += stride * CC_SILP) {
@@ -147,7 +158,7 @@ __global__ void __launch_bounds__(BLOCK)
       }
     }
 #pragma unroll
-    for (int k = 0; k < CC_SILP; ++k) (void)cc_link(a[k], b[k], p, fresh);
+    for (int k = 0; k < CC_SILP; ++k) (void)cc_link(a[k], b[k], p);
   }
 }
 
@@ -322,7 +333,7 @@ __global__ void __launch_bounds__(BLOCK)
     k_cc_rest(const int64_t *__restrict__ rows, const int32_t *__restrict__ cols,
               int64_t n, int skip_arg, const int *skip_dev,
               const int64_t *__restrict__ off, int64_t count, int *p,
-              int disjoint, bool fresh) {
+              int disjoint) {
   const int skip_root = skip_dev ? *skip_dev : skip_arg;
   const int lane = lane_id();
   const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> LOG_WAVE;
@@ -353,7 +364,7 @@ __global__ void __launch_bounds__(BLOCK)
     if (!wide)
       for (int64_t j = s; j < e; ++j) {
         const int u = cols[j];
-        if (!in_s || u < lo || u >= hi) root = cc_link(root, cc_get(p, u), p, fresh);
+        if (!in_s || u < lo || u >= hi) root = cc_link(root, cc_get(p, u), p);
       }
     uint64_t wmask = ballot(wide);
     while (wmask) {
@@ -365,7 +376,7 @@ __global__ void __launch_bounds__(BLOCK)
       int wr = __shfl(root, w, 64);
       for (int64_t j = ws + lane; j < we; j += WAVE) {
         const int u = cols[j];
-        if (!wi || u < wl || u >= wh) wr = cc_link(wr, cc_get(p, u), p, fresh);
+        if (!wi || u < wl || u >= wh) wr = cc_link(wr, cc_get(p, u), p);
       }
     }
   }

@@ -262,12 +262,14 @@ def test_cc_long_chains_and_samples(gsw, orc, shape):
 
 
 @pytest.mark.parametrize("directed", [False, True])
-@pytest.mark.parametrize("shape", ["star_last", "star_middle", "pairs", "two_hubs", "chain_of_stars",
-                                   "rmat_reversed", "rmat_half"])
+@pytest.mark.parametrize("shape", ["star_last", "star_middle", "pairs", "two_hubs", "two_hubs_first",
+                                   "eight_hubs_first", "chain_of_stars", "rmat_reversed",
+                                   "rmat_half"])
 def test_cc_hubs_anywhere(gsw, shape, directed):
     """Vertices whose only neighbour is larger (a hub with the largest id or
-    one in the middle, pairs), hubs that only second neighbours lead to, and
-    R-MAT with its hubs at the other end or with each edge in one direction."""
+    one in the middle, pairs), hubs that only second neighbours lead to, hubs
+    whose roots every lane of a wavefront hooks at once, and R-MAT with its hubs
+    at the other end or with each edge in one direction."""
     rng = np.random.default_rng(11)
     n = 5000
     if shape in ("star_last", "star_middle"):
@@ -280,6 +282,11 @@ def test_cc_hubs_anywhere(gsw, shape, directed):
     elif shape == "two_hubs":
         leaf = np.arange(n - 2)
         e = np.concatenate([np.stack([leaf, np.full(n - 2, h)], 1) for h in (n - 2, n - 1)])
+    elif shape in ("two_hubs_first", "eight_hubs_first"):
+        n, k = 70000, 2 if shape == "two_hubs_first" else 8
+        e = np.stack([np.repeat(np.arange(k), n - k), np.tile(np.arange(k, n), k)], 1)
+        if k == 8:  # each leaf under two of them
+            e = e[rng.random(len(e)) < 0.25]
     elif shape == "chain_of_stars":  # hubs last, their leaves' ids interleaved
         hub = n - 50 + np.arange(n - 50) % 50
         e = np.concatenate([np.stack([np.arange(n - 50), hub], 1),
