@@ -235,8 +235,8 @@ struct gsw_graph {
   int32_t *do_heavy = nullptr;
   int64_t *do_hpre = nullptr;
   long long *do_ctrl = nullptr;
-  long long *do_hist = nullptr;   // pinned: written by the device loop
-  long long *do_hctrl = nullptr;  // pinned copy of the first control words
+  long long *do_hist = nullptr;
+  long long *do_hctrl = nullptr;  // pinned: control words, a batch's history, mark
   hipGraph_t do_graph = nullptr;
   hipGraphExec_t do_exec = nullptr;
   double do_key[5] = {-1, -1, -1, -1, -1};
@@ -273,7 +273,7 @@ struct gsw_graph {
     if (do_heavy) hipFree(do_heavy);
     if (do_hpre) hipFree(do_hpre);
     if (do_ctrl) hipFree(do_ctrl);
-    if (do_hist) hipHostFree(do_hist);
+    if (do_hist) hipFree(do_hist);
     if (do_hctrl) hipHostFree(do_hctrl);
     if (cc_lab) hipFree(cc_lab);
     if (cc_skip) hipFree(cc_skip);
@@ -891,10 +891,9 @@ gsw::dobfs_t do_view(gsw_graph *G) {
     H_ERR(hipMalloc((void **)&G->do_heavy, sizeof(int32_t) * 2 * DO_HCAP));
     H_ERR(hipMalloc((void **)&G->do_hpre, sizeof(int64_t) * (DO_HCAP + 1)));
     H_ERR(hipMalloc((void **)&G->do_ctrl, sizeof(long long) * DO_TOTAL));
-    H_ERR(hipHostMalloc((void **)&G->do_hist, sizeof(long long) * DO_HIST * DO_HIST_W));
-    // the control words, then their mark
-    H_ERR(hipHostMalloc((void **)&G->do_hctrl, sizeof(long long) * (DO_CTRL_WORDS + 1)));
-    G->do_hctrl[DO_CTRL_WORDS] = 0;
+    H_ERR(hipMalloc((void **)&G->do_hist, sizeof(long long) * DO_HIST * DO_HIST_W));
+    H_ERR(hipHostMalloc((void **)&G->do_hctrl, sizeof(long long) * (DO_MARK + 1)));
+    G->do_hctrl[DO_MARK] = 0;
   }
   dobfs_t d;
   d.n = n;
@@ -937,7 +936,7 @@ gsw::dobfs_t do_view(gsw_graph *G) {
 int bfs_device_run(gsw_graph *G, int32_t root, int per_launch, int grid, int max_levels,
                    int64_t nroots = 0) {
   using namespace gsw;
-  GSW_REQUIRE(per_launch >= 1 && per_launch <= 256 && grid >= 1 && grid <= MAX_GRID,
+  GSW_REQUIRE(per_launch >= 1 && per_launch <= DO_MAX_LAUNCH && grid >= 1 && grid <= MAX_GRID,
               GSW_E_INVALID, "invalid device-loop shape");
   GSW_REQUIRE(root >= 0 || (nroots >= 1 && G->d_roots), E_INTERNAL_CHECK, "no roots");
   const dobfs_t d = do_view(G);
@@ -971,16 +970,20 @@ int bfs_device_run(gsw_graph *G, int32_t root, int per_launch, int grid, int max
     std::memcpy(G->do_key, key, sizeof(key));
   }
   const long long *h = G->do_hctrl;
+  std::vector<long long> hist;
   bool halted = false;
   for (int done = 0; done < max_levels && !halted; done += per_launch) {
     H_ERR(hipGraphLaunch(G->do_exec, st));
-    const long long seq = h[DO_CTRL_WORDS] + 1;
+    // the control words and the rows that this batch's levels write
+    const int rows = MIN(per_launch, MAX(0, DO_HIST - done));
+    const long long seq = h[DO_MARK] + 1;
     hipLaunchKernelGGL(k_report<long long>, dim3(1), dim3(64), 0, st,
                        (const long long *)G->do_ctrl, (int)DO_CTRL_WORDS,
-                       (const long long *)nullptr, 0, G->do_hctrl,
-                       G->do_hctrl + DO_CTRL_WORDS, seq);
+                       (const long long *)G->do_hist + (rows ? (size_t)done * DO_HIST_W : 0),
+                       rows * DO_HIST_W, G->do_hctrl, G->do_hctrl + DO_MARK, seq);
     H_ERR(hipGetLastError());
-    await_mark(h + DO_CTRL_WORDS, seq, st);
+    await_mark(h + DO_MARK, seq, st);
+    hist.insert(hist.end(), h + DO_CTRL_WORDS, h + DO_CTRL_WORDS + rows * DO_HIST_W);
     halted = h[DO_HALT] != 0;
   }
   H_ERR(hipEventRecord(G->ev1, st));
@@ -989,10 +992,10 @@ int bfs_device_run(gsw_graph *G, int32_t root, int per_launch, int grid, int max
   // are wavefront-mapped pushes over the frontier bitmap, bottom-up levels
   // thread-mapped pulls, both with the inspection folded in
   G->records.clear();
-  const int nrec = MIN(levels, DO_HIST);
+  const int nrec = MIN(levels, (int)(hist.size() / DO_HIST_W));
   if (nrec > 0) {
     for (int L = 0; L < nrec; ++L) {
-      const long long *r = G->do_hist + (size_t)L * DO_HIST_W;
+      const long long *r = hist.data() + (size_t)L * DO_HIST_W;
       gsw_level_record rec{};
       rec.level = L;
       rec.dir = r[0] ? 1 : 0;

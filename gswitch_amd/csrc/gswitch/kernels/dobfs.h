@@ -65,6 +65,7 @@ constexpr int DO_SLOTS = 64;     // partial-counter slots, one line each
 constexpr int DO_STRIDE = 16;    // long longs per slot
 constexpr int DO_DECIDE_BLOCK = 1024;
 constexpr int DO_HIST = 4096;    // levels with a history row
+constexpr int DO_MAX_LAUNCH = 256;  // levels per captured batch
 constexpr int DO_HIST_W = 4;     // direction, frontier, edges, vertices
 constexpr int DO_BU = 2;         // frontier words per wavefront step (bottom-up;
                                  // R-MAT 24 level 2: 1 word 178 us, 2 words 169 us,
@@ -90,6 +91,11 @@ enum : int {
   DO_TOTAL = DO_SLOT_BASE + DO_SLOTS * DO_STRIDE
 };
 
+// words reported to the host: the control words, a batch's history rows, the
+// mark (reported by a kernel per batch: rows stored and fenced to the host by
+// each level's decision cost a path's levels 0.5 us of 13.6)
+constexpr int DO_MARK = DO_CTRL_WORDS + DO_MAX_LAUNCH * DO_HIST_W;
+
 struct dobfs_t {
   int64_t n = 0, nw = 0, m = 0;
   const int64_t *rows = nullptr;   // out-CSR
@@ -106,7 +112,6 @@ struct dobfs_t {
   int64_t *hpre = nullptr;         // [DO_HCAP + 1] degree prefix of the list
   long long *ctrl = nullptr;       // [DO_TOTAL]
   long long *hist = nullptr;       // [DO_HIST][DO_HIST_W] per-level history
-                                   // (pinned host memory)
   int heavy_deg = 4096;            // of a found vertex
   int root_heavy = 256;            // of a root (level 0)
   float alpha = 14.f, beta = 24.f;
@@ -490,7 +495,6 @@ __global__ void __launch_bounds__(DO_DECIDE_BLOCK) k_do_decide(dobfs_t d) {
       hrow[1] = ctrl[DO_NF];
       hrow[2] = ne;
       hrow[3] = nv;
-      __threadfence_system();
     }
     if (nf == 0) {
       ctrl[DO_HALT] = 1;

@@ -259,3 +259,24 @@ def test_device_bfs_heavy_roots(gsw, orc, leaves):
             want = np.minimum(np.where(a < 0, far, a), np.where(b < 0, far, b))
             assert np.array_equal(lv, np.where(want == far, -1, want))
     g.close()
+
+
+@pytest.mark.parametrize("capture", [1, 7, 8, 256])
+@pytest.mark.parametrize("n", [2, 9, 300, 5000])
+def test_device_bfs_records_of_many_levels(gsw, capture, n):
+    """Batches that end with, before and after the search, and more levels
+    than the device history has rows (4096)."""
+    h = gsw.from_edges(n, np.arange(n - 1), np.arange(1, n))
+    g = gsw.Graph(h)
+    for root in (0, n - 1):
+        lv = g.bfs(root, capture=capture)
+        assert np.array_equal(lv, np.abs(np.arange(n) - root))
+        recs = g.records()
+        assert [r["level"] for r in recs] == list(range(min(n, 4096)))
+        assert all(r["frontier"] == 1 for r in recs)
+        deg = np.full(n, 2)
+        deg[[0, n - 1]] = 1
+        order = deg if root == 0 else deg[::-1]
+        push = [r["dir"] == "Push" for r in recs]
+        assert all(r["edges"] == order[r["level"]] for r, p in zip(recs, push) if p)
+    g.close()
