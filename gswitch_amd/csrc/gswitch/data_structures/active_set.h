@@ -126,8 +126,9 @@ __global__ void __launch_bounds__(64)
   if (s < WORK_SLOTS) row[s * WORK_SLOT_STRIDE + k] = 0;
 }
 
-// The slots of rows [0, nrows) combined into `out` (pinned host memory) and
-// cleared; one workgroup, then the mark.
+// The slots of rows [0, nrows) combined into slot 0 and `out` (pinned host
+// memory), the others cleared, so that folding again changes nothing; one
+// workgroup, then the mark.
 __global__ void __launch_bounds__(1024)
     k_work_fold(unsigned long long *base, int64_t nrows, unsigned long long *out,
                 unsigned long long *mark, unsigned long long seq) {
@@ -139,8 +140,9 @@ __global__ void __launch_bounds__(1024)
 #pragma unroll
     for (int s = 0; s < WORK_SLOTS; ++s) {
       t = sum ? t + x[s] : (x[s] > t ? x[s] : t);
-      base[s * WORK_SLOT_STRIDE + i] = 0;
+      if (s > 0) base[s * WORK_SLOT_STRIDE + i] = 0;
     }
+    base[i] = t;
     out[i] = t;
   }
   __threadfence_system();
@@ -347,7 +349,6 @@ struct active_set_t {
                        mark, seq);
     H_ERR(hipGetLastError());
     gsw::await_mark(mark, seq, st);
-    if (rows >= work_rows) work_rows = 0;
     return h_work;
   }
   // overflow state as of the last read_qsize_device (no extra sync)

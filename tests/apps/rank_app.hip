@@ -3,6 +3,7 @@
 // GSW_APP_OUT=<file> gets the read attribute (float per vertex).
 #include <cstdio>
 #include <cstdlib>
+#include <vector>
 
 #include "gswitch.h"
 
@@ -41,8 +42,9 @@ struct Rank : Functor<VC, double, float, Empty> {
   }
 };
 
-// the functor by value, as the reference's drivers take it
-template <typename Gd, typename F> void iterate(Gd g, F f, int iters) {
+// The functor by value, as the reference's drivers take it. False if the
+// records change when they are read again.
+template <typename Gd, typename F> bool iterate(Gd g, F f, int iters) {
   active_set_t as = build_active_set(g.nvertexs, conf);
   as.init();
   for (int level = 0;; ++level) {
@@ -54,6 +56,14 @@ template <typename Gd, typename F> void iterate(Gd g, F f, int iters) {
     executor.expand(as, g, f, stats, fets, conf);
     if (as.finish(g, f, conf)) break;
   }
+  executor.finalize_log(as);
+  const std::vector<level_record_t> once = executor.log;
+  executor.finalize_log(as);
+  bool same = (int)once.size() == iters;
+  for (size_t i = 0; i < once.size(); ++i)
+    same = same && once[i].edges == g.nedges && executor.log[i].edges == once[i].edges &&
+           executor.log[i].ms == once[i].ms;
+  return same;
 }
 
 int main(int argc, char *argv[]) {
@@ -79,7 +89,7 @@ int main(int argc, char *argv[]) {
   });
   init_conf(stats, fets, conf, g, f);
   const char *iters = std::getenv("GSW_APP_ITERS");
-  iterate(g.dg, f, iters ? std::atoi(iters) : 10);
+  if (!iterate(g.dg, f, iters ? std::atoi(iters) : 10)) return 2;
   f.data.sync_ra();
   if (const char *out = std::getenv("GSW_APP_OUT")) {
     FILE *fp = std::fopen(out, "wb");
