@@ -9,10 +9,11 @@
 // variant, timing history, and the fused -> standalone fallback when an
 // expand takes more than 5x the average.
 //
-// Host<->device traffic per level: standalone levels sync once (the
-// inspector's counters); fused levels sync once after the expand (the next
-// queue's length, which also tells convergence). Queue lengths are otherwise
-// known on the host from the inspector's counts.
+// Host<->device traffic per level: standalone levels wait once (the
+// inspector's counters); fused levels wait once after the expand (the next
+// queue's length, which also tells convergence), those of run_ahead() once per
+// batch of up to eight. Queue lengths are otherwise known on the host from the
+// inspector's counts.
 #pragma once
 #include <cmath>
 #include <vector>

@@ -33,8 +33,8 @@ struct ms_counters_t {
   unsigned long long pad[14];       // one slot = five 128-byte lines
 };
 // Workgroups add their counts into one of MS_SLOTS partial copies (slot
-// blockIdx.x % MS_SLOTS); the host sums the copies. Atomics that every
-// workgroup of the grid sends to the same lines serialise on MI355X.
+// blockIdx.x % MS_SLOTS); k_msbfs_finish sums and clears them. Atomics that
+// every workgroup of the grid sends to the same lines serialise on MI355X.
 constexpr int MS_SLOTS = 64;
 static_assert(sizeof(ms_counters_t) == 640, "slot size");
 

@@ -1,9 +1,9 @@
 // From-all pull of a small graph in one launch per level, the functor's
 // filter included.
 //
-// Where the sources' state fits the L2, gathering it per edge is cheaper than
-// propagation blocking's two passes over per-edge messages, whose pieces also
-// leave most of the chip idle on a small graph. Targets are listed once per
+// Where the sources' state stays in the caches, gathering it per edge is cheaper
+// than propagation blocking's two passes over per-edge messages, whose pieces
+// also leave most of the chip idle on a small graph. Targets are listed once per
 // graph by in-degree: a lane takes a row of up to 8 edges, eight lanes one of
 // up to 128, a wavefront one of up to 2048, a workgroup a longer one, so that
 // every row is summed in one place and the rank update can follow at once. The

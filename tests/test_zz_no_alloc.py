@@ -1,12 +1,12 @@
 """gsw_cc_noalloc: connected components that allocate nothing.
 
 The entry point writes the labels into a device buffer the caller owns and
-keeps its own scratch (the vertex sample and the chosen root) in a static
-device array. Its labels must equal gsw_cc's on the same graph, on two
-calls in a row whose second one is smaller (fewer vertices and fewer
-samples), with the scratch left over from the first call; and both must
-equal the oracle. The device buffers here come from the HIP runtime
-through ctypes (the test allocates; the entry point must not).
+keeps its own scratch (the chosen root) in a static device array. Its labels
+must equal gsw_cc's on the same graph, on two calls in a row whose second one
+is smaller (fewer vertices and fewer samples), with the scratch left over from
+the first call; and both must equal the oracle. The device buffers here come
+from the HIP runtime through ctypes (the test allocates; the entry point must
+not).
 """
 import ctypes as C
 
