@@ -421,6 +421,19 @@ def test_pagerank_eps_after_fixed_iterations(gsw, gset, first, eps):
     g.close()
 
 
+@pytest.mark.parametrize("configs", [None] + ["%s-Bitmap-%s-Standalone" % (d, lb)
+                                              for d in DIRS for lb in ("WM", "STRICT", "TWOD")])
+def test_pagerank_until_eps(gsw, orc, gset, configs):
+    """Runs that end once no rank changes by 1e-6 of itself: what is left to
+    the fixed point is at most 0.85 / 0.15 of that."""
+    for gname in ["rmat12", "ba", "grid"]:
+        h, g = gset[gname]
+        pr = g.pagerank(0.85, 500, eps=1e-6, configs=configs)
+        assert 5 < g.last_stats.levels < 500
+        ref = orc.pagerank(h.row_ptr, h.col, 0.85, 500)
+        assert max_rel(pr, ref) <= PR_TOL, (gname, max_rel(pr, ref))
+
+
 @pytest.mark.parametrize("configs", ["Pull-Bitmap-%s-Standalone" % lb for lb in LBS + ["TWOD"]])
 @pytest.mark.parametrize("pull_kernel", [0, 1, 2])
 def test_expand_times(gsw, gset, monkeypatch, configs, pull_kernel):
